@@ -37,6 +37,11 @@ struct DevLayer {
     uint16_t * o16 = nullptr;
     uint16_t * gu16 = nullptr;
     uint16_t * down16 = nullptr;
+    // f32 weights: their fragment-ordered three-part split for the prompt GEMMs (gemm_prefill.hip)
+    uint16_t * qkv3 = nullptr;
+    uint16_t * o3 = nullptr;
+    uint16_t * gu3 = nullptr;
+    uint16_t * down3 = nullptr;
     // q|k|v and o f32 rows packed for the multi-stream step's MFMA GEMM (gemm_packed.hip): multi-stream
     // decoders on f32 weights only
     float * qkv_p = nullptr;
@@ -75,9 +80,13 @@ struct qa_decoder {
     int32_t cap_rows = 0;
     std::vector<void *> act_allocs;
     float *x = nullptr, *xn = nullptr, *qkv = nullptr, *qrot = nullptr, *attn = nullptr, *gu = nullptr, *act = nullptr;
-    uint16_t * xsplit = nullptr;   // [rows][3 in_dim] bf16: three-part split of a GEMM input (bf16 copies)
-    size_t xsplit_elems = 0;       // a third of its size: rows x max in_dim
-    uint16_t * actsplit = nullptr; // [rows][3 intermediate] bf16: split of silu(gate) * up (fused SwiGLU)
+    // prompt projections (prompt_path): fragment-ordered splits of a GEMM input and of silu(gate) * up, K-slice
+    // partial sums, and the slices of the last down projection that are not yet in x
+    uint16_t * xf = nullptr;
+    uint16_t * actf = nullptr;
+    float * partial = nullptr;
+    size_t partial_bytes = 0;
+    int32_t pending = 0;
     float * logits = nullptr;    // [n_streams][vocab]
     void * attn_ws = nullptr;
     size_t attn_ws_bytes = 0;
@@ -174,9 +183,10 @@ void free_acts(qa_decoder * d) {
     d->pf_ws = nullptr;
     d->pf_ws_bytes = 0;
     d->xstats = nullptr;
-    d->xsplit = nullptr;
-    d->xsplit_elems = 0;
-    d->actsplit = nullptr;
+    d->xf = nullptr;
+    d->actf = nullptr;
+    d->partial = nullptr;
+    d->partial_bytes = 0;
 }
 
 // Workspace of the skinny GEMM for the layer projections at up to `rows` token rows and the LM head at
@@ -188,6 +198,19 @@ size_t gemm_rows_bytes_for(const qa_text_config & c, int32_t rows, int32_t logit
     for (const auto & sh : shapes) m = std::max(m, gemm_rows_workspace_bytes(sh[0], sh[1], rows));
     if (logit_rows >= 2) m = std::max(m, gemm_rows_workspace_bytes(c.vocab, H, logit_rows));
     return m;
+}
+
+// Whether the decoder's shapes (and, prompt_ready, its weight copies) run T > 1 prompt rows on the prompt GEMMs
+// (gemm_prefill.hip).
+bool prompt_shapes(const qa_decoder * d) {
+    const qa_text_config & c = d->cfg;
+    const int32_t H = c.hidden, QD = c.n_heads * kHeadDim, KD = c.n_kv_heads * kHeadDim, I = c.intermediate;
+    return H <= 8192 && prompt_gemm_shape_ok(QD + 2 * KD, H, false) && prompt_gemm_shape_ok(H, QD, false) &&
+           prompt_gemm_shape_ok(I, H, true) && prompt_gemm_shape_ok(H, I, false);
+}
+
+bool prompt_ready(const qa_decoder * d) {
+    return !d->layers.empty() && (d->layers[0].qkv16 || d->layers[0].qkv3) && prompt_shapes(d);
 }
 
 int ensure_rows(qa_decoder * d, int32_t rows) {
@@ -203,7 +226,7 @@ int ensure_rows(qa_decoder * d, int32_t rows) {
     rc = rc ? rc : dmalloc_t(d->act_allocs, R * (QD + 2 * KD), &d->qkv);
     rc = rc ? rc : dmalloc_t(d->act_allocs, R * QD, &d->qrot);
     rc = rc ? rc : dmalloc_t(d->act_allocs, R * QD, &d->attn);
-    rc = rc ? rc : dmalloc_t(d->act_allocs, R * 2 * I, &d->gu);
+    if (!prompt_ready(d)) rc = rc ? rc : dmalloc_t(d->act_allocs, R * 2 * I, &d->gu);
     rc = rc ? rc : dmalloc_t(d->act_allocs, R * I, &d->act);
     // the LM head runs on one row per stream (decode) or the last row (prefill)
     const size_t gr = rows >= 2 ? gemm_rows_bytes_for(d->cfg, std::min<int32_t>(rows, kSkinnyRows),
@@ -223,12 +246,11 @@ int ensure_rows(qa_decoder * d, int32_t rows) {
         const size_t n = static_cast<size_t>((H + 15) / 16) * 32;
         rc = dmalloc(d->act_allocs, n * sizeof(double), reinterpret_cast<void **>(&d->xstats));
     }
-    // bf16 copies: longer GEMM inputs are split into three bf16 parts ([rows][3 in_dim]) for the bf16 GEMM,
-    // and the fused SwiGLU writes its split output beside the gate|up input
-    if (rc == QA_OK && rows > kSkinnyRows && !d->layers.empty() && d->layers[0].qkv16) {
-        d->xsplit_elems = R * std::max({H, QD, I});
-        rc = dmalloc_t(d->act_allocs, 3 * d->xsplit_elems, &d->xsplit);
-        rc = rc ? rc : dmalloc_t(d->act_allocs, 3 * R * I, &d->actsplit);
+    if (rc == QA_OK && rows >= 2 && prompt_ready(d)) {
+        d->partial_bytes = prompt_partial_bytes(rows);
+        rc = dmalloc_t(d->act_allocs, prompt_frag_elems(rows, std::max(d->cfg.hidden, d->cfg.n_heads * kHeadDim)), &d->xf);
+        rc = rc ? rc : dmalloc_t(d->act_allocs, prompt_frag_elems(rows, d->cfg.intermediate), &d->actf);
+        rc = rc ? rc : dmalloc(d->act_allocs, d->partial_bytes, reinterpret_cast<void **>(&d->partial));
     }
     // prefill attention over up to `rows` tokens (counters cleared once; every call leaves them zero)
     const size_t pf = rows >= 2 ? qa_prefill_attn_workspace_bytes(rows, d->cfg.n_heads) : 0;
@@ -251,35 +273,12 @@ bool skinny_path(const qa_decoder * d, int32_t rows, int32_t in_dim) {
     return rows <= kSkinnyRows && in_dim % 32 == 0 && d->gr_ws;
 }
 
-// Whether sgemm runs the bf16 GEMM over the three-part split of its input (then the producer of the
-// input may write d->xsplit itself, see sgemm's x_split).  W16: the bf16 rows; swiglu: the fused SwiGLU
-// GEMM (out_dim = intermediate, W16 = [gate rows; up rows]).
-bool split_path(const qa_decoder * d, int32_t rows, int32_t out_dim, int32_t in_dim, const uint16_t * W16,
-                bool swiglu = false) {
-    return !skinny_path(d, rows, in_dim) && W16 && d->xsplit && static_cast<size_t>(rows) * in_dim <= d->xsplit_elems &&
-           gemm_split3_shape_ok(out_dim, in_dim, swiglu);
-}
-
 int sgemm(qa_decoder * d, const float * W, int32_t out_dim, int32_t in_dim, const float * X, int32_t rows, float * Y,
-          float beta, const uint16_t * W16 = nullptr, const uint16_t * x_split = nullptr) {
-    // Y[rows][out] (+)= X[rows][in] * W[out][in]^T.  Up to kSkinnyRows rows (multi-stream decode, short
-    // prefills) the weights are streamed once by the skinny MFMA GEMM; longer prefills run gemm_split3 on
-    // the bf16 copies, or rocBLAS sgemm on f32 weights.  x_split: the producer of X already wrote its
-    // three-part split there (only where split_path holds).
-    if (x_split && !split_path(d, rows, out_dim, in_dim, W16)) {
-        return fail(QA_ERR_INVALID, "sgemm: split input without split path");
-    }
+          float beta) {
+    // Y[rows][out] (+)= X[rows][in] * W[out][in]^T on f32 weights.  Up to kSkinnyRows rows (multi-stream decode,
+    // short prefills) the weights are streamed once by the skinny MFMA GEMM; longer prefills run rocBLAS sgemm.
     if (skinny_path(d, rows, in_dim)) {
         return gemm_rows_launch(W, out_dim, in_dim, X, rows, Y, beta != 0.0f, d->gr_ws, d->gr_ws_bytes, d->stream);
-    }
-    if (split_path(d, rows, out_dim, in_dim, W16)) {
-        // bf16-exact weights: each row of X split into three bf16 parts, X = hi + mid + lo exactly, and one
-        // bf16 MFMA GEMM over the one bf16 copy uses every W tile for the three parts: every product exact,
-        // the sums in f32 (gemm_split3.hip)
-        const int rc = x_split ? QA_OK : split_bf16x3_rows_launch(X, rows, in_dim, d->xsplit, d->stream);
-        if (rc != QA_OK) return rc;
-        return gemm_split3_launch(W16, out_dim, in_dim, x_split ? x_split : d->xsplit, rows, Y, beta != 0.0f, nullptr,
-                                  d->stream);
     }
     // column-major C(out x rows) = W^T(out x in) * X(in x rows)
     const float alpha = 1.0f;
@@ -330,6 +329,24 @@ int32_t host_max_len(const qa_decoder * d, int32_t n, int32_t add) {
     return m;
 }
 
+// One projection of the prompt path: W [N][K] (act: [gate; up] of N outputs) times the split input Xf.
+int prompt_gemm(qa_decoder * d, const uint16_t * W16, const uint16_t * W3, int32_t N, int32_t K, const uint16_t * Xf, int32_t rows, float * Y,
+                bool accumulate, uint16_t * act, int32_t * slices) {
+    PromptGemm g;
+    g.Xf = Xf;
+    g.W16 = W16;
+    g.W3 = W3;
+    g.Y = Y;
+    g.act = act;
+    g.partial = d->partial;
+    g.partial_bytes = d->partial_bytes;
+    g.M = rows;
+    g.N = N;
+    g.K = K;
+    g.accumulate = accumulate;
+    return prompt_gemm_launch(g, slices, d->stream);
+}
+
 // One layer over `rows` token rows held in d->x.
 //   kDecode : rows = number of streams (one token each), positions d_lens[s], keys [0, d_lens[s] + 1)
 //   kPrefill: rows = T tokens of stream 0 at positions n_past.., keys [0, n_past + t]
@@ -341,10 +358,17 @@ int run_layer(qa_decoder * d, int32_t l, int32_t rows, int kind, int32_t n_past,
     const int32_t H = c.hidden, QD = c.n_heads * kHeadDim, KD = c.n_kv_heads * kHeadDim, I = c.intermediate;
     const int32_t W3 = QD + 2 * KD;
     hipStream_t s = d->stream;
+    const bool prompt = rows > 1 && !fused && d->xf;
+    int32_t slices = 0;   // K slices of the q|k|v projection, still partial sums in d->partial
     int rc;
     {
         Prof pr(d, kFamProj);
-        if (rows == 1) {
+        if (prompt) {
+            rc = prompt_norm_launch(d->x, d->partial, d->pending, L.attn_norm, rows, H, c.rms_norm_eps, d->xf, s);
+            d->pending = 0;
+            if (rc == QA_OK) rc = prompt_gemm(d, L.qkv16, L.qkv3, W3, H, d->xf, rows, d->qkv, false, nullptr, &slices);
+            if (rc == QA_OK && slices > 0 && kind != kPrefill) rc = prompt_sum_launch(d->partial, slices, rows, W3, d->qkv, s);
+        } else if (rows == 1) {
             rc = gemv_launch(kEpiStoreOp, true, L.qkv, W3, H, d->x, d->qkv, L.attn_norm, c.rms_norm_eps, s,
                              L.qkv16);
         } else if (fused) {
@@ -352,10 +376,8 @@ int run_layer(qa_decoder * d, int32_t l, int32_t rows, int kind, int32_t n_past,
             rc = L.qkv_p ? gemm_packed_launch(L.qkv_p, W3, H, d->x, rows, d->qkv, false, &f, false, s)
                          : fused_gemm(d, L.qkv, W3, H, d->x, rows, d->qkv, false, f, L.qkv16);
         } else {
-            // the RMSNorm writes the GEMM's split input directly where the GEMM takes one
-            const bool sp = split_path(d, rows, W3, H, L.qkv16);
-            rc = rmsnorm_rows_launch(d->x, L.attn_norm, rows, H, c.rms_norm_eps, d->xn, s, sp ? d->xsplit : nullptr);
-            if (rc == QA_OK) rc = sgemm(d, L.qkv, W3, H, d->xn, rows, d->qkv, 0.0f, L.qkv16, sp ? d->xsplit : nullptr);
+            rc = rmsnorm_rows_launch(d->x, L.attn_norm, rows, H, c.rms_norm_eps, d->xn, s);
+            if (rc == QA_OK) rc = sgemm(d, L.qkv, W3, H, d->xn, rows, d->qkv, 0.0f);
         }
         if (rc != QA_OK) return rc;
     }
@@ -380,8 +402,8 @@ int run_layer(qa_decoder * d, int32_t l, int32_t rows, int kind, int32_t n_past,
     } else {
         {
             Prof pr(d, kFamAppend);
-            rc = qa_kv_append(d->qkv, L.q_norm, L.k_norm, d->qrot, d->cache, &d->layout, l, d->d_lens, 1, rows,
-                              c.n_heads, c.rope_theta, c.rms_norm_eps, s);
+            rc = kv_append_launch(slices > 0 ? d->partial : d->qkv, slices, L.q_norm, L.k_norm, d->qrot, d->cache,
+                                  d->layout, l, d->d_lens, 1, rows, c.n_heads, c.rope_theta, c.rms_norm_eps, s);
             if (rc != QA_OK) return rc;
         }
         Prof pr(d, kFamPrefillAttn);
@@ -390,7 +412,15 @@ int run_layer(qa_decoder * d, int32_t l, int32_t rows, int kind, int32_t n_past,
         if (rc != QA_OK) return rc;
     }
     Prof pr(d, kFamProj);
-    if (rows == 1) {
+    if (prompt) {
+        int32_t po = 0, pg = 0;
+        rc = prompt_split_launch(d->attn, rows, QD, d->xf, s);
+        if (rc == QA_OK) rc = prompt_gemm(d, L.o16, L.o3, H, QD, d->xf, rows, d->x, true, nullptr, &po);
+        if (rc == QA_OK) rc = prompt_norm_launch(d->x, d->partial, po, L.ffn_norm, rows, H, c.rms_norm_eps, d->xf, s);
+        if (rc == QA_OK) rc = prompt_gemm(d, L.gu16, L.gu3, I, H, d->xf, rows, nullptr, false, d->actf, &pg);
+        if (rc == QA_OK && pg > 0) rc = prompt_swiglu_launch(d->partial, pg, rows, I, d->actf, s);
+        if (rc == QA_OK) rc = prompt_gemm(d, L.down16, L.down3, H, I, d->actf, rows, d->x, true, nullptr, &d->pending);
+    } else if (rows == 1) {
         rc = gemv_launch(kEpiAccumOp, false, L.o, H, QD, d->attn, d->x, nullptr, 0.0f, s, L.o16);
         if (rc == QA_OK) {
             rc = gemv_launch(kEpiSwigluOp, true, L.gu, I, H, d->x, d->act, L.ffn_norm, c.rms_norm_eps, s, L.gu16);
@@ -409,21 +439,27 @@ int run_layer(qa_decoder * d, int32_t l, int32_t rows, int kind, int32_t n_past,
         if (rc == QA_OK) rc = fused_gemm(d, L.gu, 2 * I, H, d->x, rows, d->act, false, gu, L.gu16);
         if (rc == QA_OK) rc = fused_gemm(d, L.down, H, I, d->act, rows, d->x, true, stats_out(d), L.down16);
     } else {
-        rc = sgemm(d, L.o, H, QD, d->attn, rows, d->x, 1.0f, L.o16);
-        const bool sd = split_path(d, rows, H, I, L.down16) && d->actsplit;
-        // bf16 copies: gate|up with the SwiGLU in its epilogue, writing the split input of down directly
-        const bool fuse = sd && split_path(d, rows, I, H, L.gu16, true);
-        const bool sg = fuse || split_path(d, rows, 2 * I, H, L.gu16);
-        if (rc == QA_OK) rc = rmsnorm_rows_launch(d->x, L.ffn_norm, rows, H, c.rms_norm_eps, d->xn, s, sg ? d->xsplit : nullptr);
-        if (fuse) {
-            if (rc == QA_OK) rc = gemm_split3_launch(L.gu16, I, H, d->xsplit, rows, nullptr, false, d->actsplit, s);
-        } else {
-            if (rc == QA_OK) rc = sgemm(d, L.gu, 2 * I, H, d->xn, rows, d->gu, 0.0f, L.gu16, sg ? d->xsplit : nullptr);
-            if (rc == QA_OK) rc = swiglu_rows_launch(d->gu, rows, I, d->act, s, sd ? d->actsplit : nullptr);
-        }
-        if (rc == QA_OK) rc = sgemm(d, L.down, H, I, d->act, rows, d->x, 1.0f, L.down16, sd ? d->actsplit : nullptr);
+        rc = sgemm(d, L.o, H, QD, d->attn, rows, d->x, 1.0f);
+        if (rc == QA_OK) rc = rmsnorm_rows_launch(d->x, L.ffn_norm, rows, H, c.rms_norm_eps, d->xn, s);
+        if (rc == QA_OK) rc = sgemm(d, L.gu, 2 * I, H, d->xn, rows, d->gu, 0.0f);
+        if (rc == QA_OK) rc = swiglu_rows_launch(d->gu, rows, I, d->act, s);
+        if (rc == QA_OK) rc = sgemm(d, L.down, H, I, d->act, rows, d->x, 1.0f);
     }
     return rc;
+}
+
+// Layers first .. last - 1; the last down projection's partial sums, which the next layer's RMSNorm would add, are
+// added to x at the end.
+int run_layers(qa_decoder * d, int32_t first, int32_t last, int32_t rows, int kind, int32_t n_past, int32_t max_len = 0,
+               bool fused = false) {
+    d->pending = 0;
+    for (int32_t l = first; l < last; ++l) {
+        const int rc = run_layer(d, l, rows, kind, n_past, max_len, fused);
+        if (rc != QA_OK) return rc;
+    }
+    if (d->pending == 0) return QA_OK;
+    Prof pr(d, kFamProj);
+    return prompt_norm_launch(d->x, d->partial, d->pending, nullptr, rows, d->cfg.hidden, 0.0f, nullptr, d->stream);
 }
 
 // Logits of `rows` rows starting at row `first` of d->x into d->logits[0..rows), then greedy ids.
@@ -527,10 +563,8 @@ int forward_device(qa_decoder * d, int32_t n_tokens, int32_t n_past, bool pick) 
         rc = persist_layers(d, n_past + 1);
         if (rc != QA_OK) return rc;
     } else {
-        for (int32_t l = 0; l < d->cfg.n_layers; ++l) {
-            rc = run_layer(d, l, n_tokens, kind, n_past);
-            if (rc != QA_OK) return rc;
-        }
+        rc = run_layers(d, 0, d->cfg.n_layers, n_tokens, kind, n_past);
+        if (rc != QA_OK) return rc;
     }
     rc = logits_and_pick(d, n_tokens - 1, 1, pick);
     if (rc != QA_OK) return rc;
@@ -553,10 +587,8 @@ int decode_step_ops(qa_decoder * d, int32_t rows, int32_t max_len, bool embed, i
     }
     if (d->persist && rows == 1) {
         if (rc == QA_OK) rc = persist_layers(d, max_len);
-    } else {
-        for (int32_t l = 0; l < d->cfg.n_layers && rc == QA_OK; ++l) {
-            rc = run_layer(d, l, rows, kDecode, 0, max_len, fused);
-        }
+    } else if (rc == QA_OK) {
+        rc = run_layers(d, 0, d->cfg.n_layers, rows, kDecode, 0, max_len, fused);
     }
     StepTail tail;
     tail.lens = d->d_lens;
@@ -623,6 +655,38 @@ int pack_weights_bf16(qa_decoder * d) {
         for (DevLayer & L : d->layers) L.qkv16 = L.o16 = L.gu16 = L.down16 = nullptr;
         d->out_w16 = nullptr;
     }
+    return rc;
+}
+
+// f32 weights: the three-part split of every projection in fragment order, 6 bytes per weight (8.5 GB for the 1.7B
+// model), with which a prompt's projections run on bf16 MFMA: 1.6 times rocBLAS sgemm's speed at T = 3913.  Laid out
+// once, since splitting W in the GEMM would repeat it for every token group, and a pass per call would move ten bytes
+// per weight (90 us beside 126 us of GEMMs per 1.7B layer at T = 156).  Without the memory the prompts keep sgemm.
+int pack_weights_prompt(qa_decoder * d) {
+    if (d->layers.empty() || d->layers[0].qkv16 || !prompt_shapes(d)) return QA_OK;
+    const qa_text_config & c = d->cfg;
+    const int32_t H = c.hidden, QD = c.n_heads * kHeadDim, KD = c.n_kv_heads * kHeadDim, I = c.intermediate;
+    std::vector<void *> allocs;
+    int rc = QA_OK;
+    auto pack = [&](const float * src, int32_t N, int32_t K, uint16_t ** dst) {
+        if (rc != QA_OK) return;
+        rc = dmalloc_t(allocs, prompt_frag_elems(N, K), dst);
+        if (rc == QA_OK) rc = prompt_split_launch(src, N, K, *dst, d->stream);
+    };
+    for (DevLayer & L : d->layers) {
+        pack(L.qkv, QD + 2 * KD, H, &L.qkv3);
+        pack(L.o, H, QD, &L.o3);
+        pack(L.gu, 2 * I, H, &L.gu3);
+        pack(L.down, H, I, &L.down3);
+    }
+    if (rc == QA_ERR_ALLOC) {
+        (void)hipGetLastError();
+        (void)hipStreamSynchronize(d->stream);
+        for (void * p : allocs) (void)hipFree(p);
+        for (DevLayer & L : d->layers) L.qkv3 = L.o3 = L.gu3 = L.down3 = nullptr;
+        return QA_OK;
+    }
+    d->weight_allocs.insert(d->weight_allocs.end(), allocs.begin(), allocs.end());
     return rc;
 }
 
@@ -746,6 +810,7 @@ extern "C" int qa_decoder_create(const qa_text_config * cfg, const qa_model_weig
     if (rc != QA_OK) return bail(rc);
     rc = pack_weights_bf16(d);
     if (rc == QA_OK) rc = pack_weights_mfma(d);
+    if (rc == QA_OK) rc = pack_weights_prompt(d);
     if (rc != QA_OK) return bail(rc);
 
     d->layout.n_layers = cfg->n_layers;
@@ -1065,7 +1130,7 @@ extern "C" int qa_decoder_layer_forward(qa_decoder * d, int32_t layer, const flo
     QA_HIP(hipMemcpyAsync(d->x, x, sizeof(float) * n_tokens * d->cfg.hidden, hipMemcpyHostToDevice, d->stream));
     rc = set_values_launch(d->d_lens, 1, n_past, d->stream);
     d->cur_len[0] = n_past;
-    if (rc == QA_OK) rc = run_layer(d, layer, n_tokens, n_tokens == 1 ? kDecode : kPrefill, n_past);
+    if (rc == QA_OK) rc = run_layers(d, layer, layer + 1, n_tokens, n_tokens == 1 ? kDecode : kPrefill, n_past);
     if (rc == QA_OK) rc = set_values_launch(d->d_lens, 1, n_past + n_tokens, d->stream);
     if (rc != QA_OK) return rc;
     d->cur_len[0] = n_past + n_tokens;
@@ -1082,7 +1147,7 @@ extern "C" int qa_decoder_layer_forward_nocache(qa_decoder * d, int32_t layer, c
     int rc = ensure_rows(d, n_tokens);
     if (rc != QA_OK) return rc;
     QA_HIP(hipMemcpyAsync(d->x, x, sizeof(float) * n_tokens * d->cfg.hidden, hipMemcpyHostToDevice, d->stream));
-    rc = run_layer(d, layer, n_tokens, kNoCache, 0);
+    rc = run_layers(d, layer, layer + 1, n_tokens, kNoCache, 0);
     if (rc != QA_OK) return rc;
     QA_HIP(hipMemcpyAsync(y, d->x, sizeof(float) * n_tokens * d->cfg.hidden, hipMemcpyDeviceToHost, d->stream));
     QA_HIP(hipStreamSynchronize(d->stream));
@@ -1094,7 +1159,7 @@ extern "C" int qa_decoder_prefill_nocache(qa_decoder * d, const float * x, int32
     int rc = ensure_rows(d, n_tokens);
     if (rc != QA_OK) return rc;
     QA_HIP(hipMemcpyAsync(d->x, x, sizeof(float) * n_tokens * d->cfg.hidden, hipMemcpyHostToDevice, d->stream));
-    for (int32_t l = 0; l < d->cfg.n_layers && rc == QA_OK; ++l) rc = run_layer(d, l, n_tokens, kNoCache, 0);
+    rc = run_layers(d, 0, d->cfg.n_layers, n_tokens, kNoCache, 0);
     if (rc == QA_OK) rc = logits_and_pick(d, n_tokens - 1, 1, false);
     if (rc != QA_OK) return rc;
     QA_HIP(hipMemcpyAsync(logits, d->logits, sizeof(float) * d->cfg.vocab, hipMemcpyDeviceToHost, d->stream));

@@ -13,7 +13,6 @@
 // products and sums are the f32 kernel's, operation for operation, at half the bytes.
 #include "gemv_body.hpp"
 #include "ops.hpp"
-#include "split3.hpp"
 #include "wave.hpp"
 
 #include <algorithm>
@@ -790,10 +789,9 @@ GemmRowsPlan gemm_rows_plan(int32_t N, int32_t K, int32_t rows, bool one_slice =
 }
 
 // ---------------------------------------------------------------- row RMSNorm (T > 1 paths)
-// y = RMSNorm(x) w per row, as f32 rows of y or (split != null) as the three-part split rows of the
-// prefill GEMM's input ([rows][3 dim] bf16 bits)
+// y = RMSNorm(x) w per row
 __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const float * x, const float * w, int dim, float eps,
-                                                           float * y, uint16_t * split) {
+                                                           float * y) {
 #pragma clang fp contract(off)
     const int r = blockIdx.x;
     const float * xr = x + static_cast<int64_t>(r) * dim;
@@ -805,27 +803,19 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const float * x, cons
     __syncthreads();
     const double tot = (part[0] + part[1]) + (part[2] + part[3]);
     const float scale = 1.0f / sqrtf(static_cast<float>(tot / static_cast<double>(dim)) + eps);
-    if (split) {
-        uint16_t * sr = split + static_cast<int64_t>(r) * 3 * dim;
-        for (int i = threadIdx.x; i < dim; i += 256) store_split3(sr + i, dim, xr[i] * scale * w[i]);
-        return;
-    }
     float * yr = y + static_cast<int64_t>(r) * dim;
     for (int i = threadIdx.x; i < dim; i += 256) yr[i] = xr[i] * scale * w[i];
 }
 
-// a = silu(gate) up per row (gu rows = [gate | up], dim each), text-decoder.cpp:602; as f32 rows of a or
-// (split != null) as the three-part split rows of the prefill GEMM's input.  blockIdx.y = row.
-__global__ __launch_bounds__(256) void swiglu_rows_kernel(const float * gu, int dim, float * a, uint16_t * split) {
+// a = silu(gate) up per row (gu rows = [gate | up], dim each), text-decoder.cpp:602.  blockIdx.y = row.
+__global__ __launch_bounds__(256) void swiglu_rows_kernel(const float * gu, int dim, float * a) {
 #pragma clang fp contract(off)
     const int c = static_cast<int>(blockIdx.x) * 256 + static_cast<int>(threadIdx.x);
     if (c >= dim) return;
     const int64_t r = blockIdx.y;
     const float g = gu[r * 2 * dim + c];
     const float u = gu[r * 2 * dim + dim + c];
-    const float v = (g / (1.0f + expf(-g))) * u;
-    if (split) store_split3(split + r * 3 * dim + c, dim, v);
-    else a[r * dim + c] = v;
+    a[r * dim + c] = (g / (1.0f + expf(-g))) * u;
 }
 
 __global__ void add_inplace_kernel(float * y, const float * x, size_t n) {
@@ -1009,42 +999,6 @@ int gemv_launch(int epi, bool prenorm, const float * W, int32_t out_dim, int32_t
     return prenorm ? launch_gemv_w<kEpiSwiglu, true>(p, b16, stream) : launch_gemv_w<kEpiSwiglu, false>(p, b16, stream);
 }
 
-// Row t of out = [hi | mid | lo] of row t of x (rows x K floats): the exact three-part bf16 split,
-// x = hi + mid + lo (truncations to 8 significant bits, then the same of the remainder; the last
-// remainder has at most 8 significant bits).  blockIdx.y = row, 4 consecutive elements per thread.
-__device__ inline uint32_t split3_pair(float a, float b, uint32_t & mid, uint32_t & lo) {
-    const uint32_t ha = __float_as_uint(a) & 0xffff0000u, hb = __float_as_uint(b) & 0xffff0000u;
-    const float ra = a - __uint_as_float(ha), rb = b - __uint_as_float(hb);
-    const uint32_t ma = __float_as_uint(ra) & 0xffff0000u, mb = __float_as_uint(rb) & 0xffff0000u;
-    const float qa = ra - __uint_as_float(ma), qb = rb - __uint_as_float(mb);
-    mid = (ma >> 16) | mb;
-    lo = (__float_as_uint(qa) >> 16) | (__float_as_uint(qb) & 0xffff0000u);
-    return (ha >> 16) | hb;
-}
-
-__global__ __launch_bounds__(256) void split_bf16x3_rows_kernel(const float * x, int32_t K, uint16_t * out) {
-    const int k = (static_cast<int>(blockIdx.x) * 256 + static_cast<int>(threadIdx.x)) * 4;
-    if (k >= K) return;
-    const int64_t t = blockIdx.y;
-    const float4 v = *reinterpret_cast<const float4 *>(x + t * K + k);
-    uint32_t m0, m1, l0, l1;
-    const uint32_t h0 = split3_pair(v.x, v.y, m0, l0), h1 = split3_pair(v.z, v.w, m1, l1);
-    uint16_t * o = out + t * 3 * K + k;
-    *reinterpret_cast<uint2 *>(o) = make_uint2(h0, h1);
-    *reinterpret_cast<uint2 *>(o + K) = make_uint2(m0, m1);
-    *reinterpret_cast<uint2 *>(o + 2 * K) = make_uint2(l0, l1);
-}
-
-int split_bf16x3_rows_launch(const float * x, int64_t rows, int32_t K, uint16_t * out, hipStream_t stream) {
-    if (!x || !out || rows < 0 || K <= 0 || K % 4 != 0) return fail(QA_ERR_INVALID, "split_bf16x3_rows: invalid arguments");
-    for (int64_t r0 = 0; r0 < rows; r0 += 65535) {     // grid.y <= 65535 rows per launch
-        const dim3 grid(static_cast<unsigned>((K / 4 + 255) / 256), static_cast<unsigned>(std::min<int64_t>(rows - r0, 65535)));
-        hipLaunchKernelGGL(split_bf16x3_rows_kernel, grid, dim3(256), 0, stream, x + r0 * K, K, out + r0 * 3 * K);
-        QA_LAUNCH_CHECK("split_bf16x3_rows_kernel");
-    }
-    return QA_OK;
-}
-
 int pack_bf16_launch(const float * src, int64_t n, uint16_t * dst, uint32_t * inexact, hipStream_t stream) {
     if (!src || !dst || !inexact || n < 0) return fail(QA_ERR_INVALID, "pack_bf16: invalid arguments");
     if (n == 0) return QA_OK;
@@ -1161,21 +1115,20 @@ int argmax_launch(const float * logits, int32_t rows, int32_t vocab, int32_t * i
 }
 
 int rmsnorm_rows_launch(const float * x, const float * w, int32_t rows, int32_t dim, float eps, float * y,
-                        hipStream_t stream, uint16_t * split) {
+                        hipStream_t stream) {
     if (rows <= 0) return QA_OK;
     hipLaunchKernelGGL(rmsnorm_rows_kernel, dim3(static_cast<unsigned>(rows)), dim3(256), 0, stream, x, w, dim,
-                       eps, y, split);
+                       eps, y);
     QA_LAUNCH_CHECK("rmsnorm_rows_kernel");
     return QA_OK;
 }
 
-int swiglu_rows_launch(const float * gu, int32_t rows, int32_t dim, float * a, hipStream_t stream, uint16_t * split) {
+int swiglu_rows_launch(const float * gu, int32_t rows, int32_t dim, float * a, hipStream_t stream) {
     if (rows <= 0 || dim <= 0) return QA_OK;
     for (int32_t r0 = 0; r0 < rows; r0 += 65535) {     // grid.y <= 65535 rows per launch
         const dim3 grid(static_cast<unsigned>((dim + 255) / 256), static_cast<unsigned>(std::min(rows - r0, 65535)));
         const int64_t off = static_cast<int64_t>(r0) * dim;
-        hipLaunchKernelGGL(swiglu_rows_kernel, grid, dim3(256), 0, stream, gu + 2 * off, dim, split ? nullptr : a + off,
-                           split ? split + 3 * off : nullptr);
+        hipLaunchKernelGGL(swiglu_rows_kernel, grid, dim3(256), 0, stream, gu + 2 * off, dim, a + off);
         QA_LAUNCH_CHECK("swiglu_rows_kernel");
     }
     return QA_OK;

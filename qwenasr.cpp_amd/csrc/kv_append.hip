@@ -37,12 +37,14 @@ struct PrepParams {
     int32_t pos0;             //                          (in-place mode)
     int32_t n_rows, n_tokens, n_heads, n_kv_heads, n_streams, max_seq, layer;
     float eps;
+    int32_t slices;           // > 0: qkv is the sum over [slices][n_rows][q_dim + 2 kv_dim], in order (cache modes)
 };
 
 // One workgroup per token row; wave w prepares the head slots w, w + 4, w + 8, ... of the row (q heads,
 // then k heads, then v heads).  The RoPE angles depend only on the position, so each wave evaluates
 // its lane's cos/sin once for all of its q and k heads.  Every load of a group of 8 slots is issued
-// before the first arithmetic; slots past the end re-read the last slot and are not stored.
+// before the first arithmetic; slots past the end re-read the last slot and are not stored.  With slices > 0 the row
+// is the sum of a projection's partial sums, so that no pass over them of its own is needed.
 template <int MODE>
 __global__ __launch_bounds__(256) void qkv_prep_kernel(PrepParams p, RopeTable rope) {
 #pragma clang fp contract(off)
@@ -65,12 +67,33 @@ __global__ __launch_bounds__(256) void qkv_prep_kernel(PrepParams p, RopeTable r
     const float wka = p.k_norm_w[lane], wkb = p.k_norm_w[lane + 64];
     constexpr int kPer = 8;
     float a[kPer], b[kPer];
+    auto load_slots = [&](int s0) {
 #pragma unroll
-    for (int u = 0; u < kPer; ++u) {
-        const int slot = min(wave + 4 * u, slots - 1);
-        a[u] = src_row[slot * kHeadDim + lane];
-        b[u] = src_row[slot * kHeadDim + lane + 64];
-    }
+        for (int u = 0; u < kPer; ++u) {
+            const int slot = min(s0 + 4 * u, slots - 1);
+            a[u] = src_row[slot * kHeadDim + lane];
+            b[u] = src_row[slot * kHeadDim + lane + 64];
+        }
+        if (MODE == kPrepInPlace) return;
+        const float * q = src_row;
+#pragma unroll 2
+        for (int s = 1; s < p.slices; ++s) {
+            q += static_cast<int64_t>(p.n_rows) * row_width;
+            float c[kPer], d[kPer];
+#pragma unroll
+            for (int u = 0; u < kPer; ++u) {
+                const int slot = min(s0 + 4 * u, slots - 1);
+                c[u] = q[slot * kHeadDim + lane];
+                d[u] = q[slot * kHeadDim + lane + 64];
+            }
+#pragma unroll
+            for (int u = 0; u < kPer; ++u) {
+                a[u] += c[u];
+                b[u] += d[u];
+            }
+        }
+    };
+    load_slots(wave);
     float c, s;
     rope_cos_sin(pos, inv_freq, c, s);
     for (int s0 = wave;; s0 += 4 * kPer) {
@@ -111,13 +134,7 @@ __global__ __launch_bounds__(256) void qkv_prep_kernel(PrepParams p, RopeTable r
             }
         }
         if (s0 + 4 * kPer >= slots) break;
-        // next group of slots (more than 32 head slots per row)
-#pragma unroll
-        for (int u = 0; u < kPer; ++u) {
-            const int slot = min(s0 + 4 * kPer + 4 * u, slots - 1);
-            a[u] = src_row[slot * kHeadDim + lane];
-            b[u] = src_row[slot * kHeadDim + lane + 64];
-        }
+        load_slots(s0 + 4 * kPer);   // more than 32 head slots per row
     }
 }
 
@@ -136,6 +153,29 @@ int launch_prep(int mode, const PrepParams & p, float rope_theta, hipStream_t st
 }
 
 }  // namespace
+
+int kv_append_launch(const float * qkv, int32_t slices, const float * q_norm_w, const float * k_norm_w, float * q_out,
+                     void * cache, const qa_kv_layout & layout, int32_t layer, const int32_t * n_past, int32_t n_streams,
+                     int32_t n_tokens, int32_t n_heads, float rope_theta, float eps, hipStream_t stream) {
+    PrepParams p{};
+    p.qkv = const_cast<float *>(qkv);
+    p.slices = slices;
+    p.q_norm_w = q_norm_w;
+    p.k_norm_w = k_norm_w;
+    p.q_out = q_out;
+    p.cache = cache;
+    p.n_past = n_past;
+    p.n_rows = n_streams * n_tokens;
+    p.n_tokens = n_tokens;
+    p.n_heads = n_heads;
+    p.n_kv_heads = layout.n_kv_heads;
+    p.n_streams = layout.n_streams;
+    p.max_seq = layout.max_seq;
+    p.layer = layer;
+    p.eps = eps;
+    return launch_prep(layout.cache_type == QA_CACHE_F16 ? kPrepCacheF16 : kPrepCacheF32, p, rope_theta, stream);
+}
+
 }  // namespace qa
 
 extern "C" int qa_kv_append(const float * qkv, const float * q_norm_w, const float * k_norm_w,
@@ -151,23 +191,8 @@ extern "C" int qa_kv_append(const float * qkv, const float * q_norm_w, const flo
         n_streams > layout->n_streams || n_tokens <= 0 || n_heads <= 0 || n_heads % layout->n_kv_heads != 0) {
         return fail(QA_ERR_INVALID, "qa_kv_append: invalid shape");
     }
-    PrepParams p{};
-    p.qkv = const_cast<float *>(qkv);
-    p.q_norm_w = q_norm_w;
-    p.k_norm_w = k_norm_w;
-    p.q_out = q_out;
-    p.cache = cache;
-    p.n_past = n_past;
-    p.n_rows = n_streams * n_tokens;
-    p.n_tokens = n_tokens;
-    p.n_heads = n_heads;
-    p.n_kv_heads = layout->n_kv_heads;
-    p.n_streams = layout->n_streams;
-    p.max_seq = layout->max_seq;
-    p.layer = layer;
-    p.eps = eps;
-    return launch_prep(layout->cache_type == QA_CACHE_F16 ? kPrepCacheF16 : kPrepCacheF32, p, rope_theta,
-                       as_stream(stream));
+    return kv_append_launch(qkv, 0, q_norm_w, k_norm_w, q_out, cache, *layout, layer, n_past, n_streams, n_tokens, n_heads,
+                            rope_theta, eps, as_stream(stream));
 }
 
 extern "C" int qa_qk_prep(float * qkv, int32_t n_tokens, int32_t n_heads, int32_t n_kv_heads,

@@ -10,8 +10,34 @@ enum { kEpiStoreOp = 0, kEpiAccumOp = 1, kEpiSwigluOp = 2 };
 // W16 (optional): the same weights as bf16 bits, read instead of W when given (bf16-exact weights)
 int gemv_launch(int epi, bool prenorm, const float * W, int32_t out_dim, int32_t in_dim, const float * x, float * y,
                 const float * norm_w, float eps, hipStream_t stream, const uint16_t * W16 = nullptr);
-// out[t] = [hi | mid | lo] of x[t] (rows x K): the exact three-part bf16 split, x = hi + mid + lo (bf16 bits)
-int split_bf16x3_rows_launch(const float * x, int64_t rows, int32_t K, uint16_t * out, hipStream_t stream);
+// Prompt projections (gemm_prefill.hip): Y[M][N] (+)= X[M][K] W[N][K]^T, X given as its fragment-ordered three-part
+// split (prompt_frag_elems bf16 values), W as the bf16 bits of bf16-exact weights (W16) or as the same split of f32
+// weights (W3, prompt_split_launch of their rows); with act != nullptr W = [gate rows; up rows]
+// (2 N rows) and act receives the fragment-ordered split of silu(gate) * up.  *slices = 0: done; otherwise the
+// *slices K slices' partial sums [slices][M][W rows] lie in `partial` and the next row kernel adds them up.
+struct PromptGemm {
+    const uint16_t * Xf = nullptr;
+    const uint16_t * W16 = nullptr;
+    const uint16_t * W3 = nullptr;   // read when W16 is null
+    float * Y = nullptr;
+    uint16_t * act = nullptr;
+    float * partial = nullptr;
+    size_t partial_bytes = 0;       // prompt_partial_bytes(rows) holds every plan of at most `rows` rows
+    int32_t M = 0, N = 0, K = 0;
+    bool accumulate = false;        // Y += (without K slices; with them the row kernel adds)
+};
+bool prompt_gemm_shape_ok(int32_t N, int32_t K, bool swiglu);
+size_t prompt_partial_bytes(int32_t rows);
+size_t prompt_frag_elems(int32_t rows, int32_t K);
+int prompt_gemm_launch(const PromptGemm & g, int32_t * slices, hipStream_t stream);
+// x += partial sums (slices > 0), then (Xf != null) Xf = the split of RMSNorm(x) w; dim % 16 == 0, dim <= 8192
+int prompt_norm_launch(float * x, const float * partial, int32_t slices, const float * w, int32_t rows, int32_t dim,
+                       float eps, uint16_t * Xf, hipStream_t stream);
+int prompt_split_launch(const float * x, int32_t rows, int32_t dim, uint16_t * Xf, hipStream_t stream);
+// Xf = the split of silu(gate) up, gate | up summed over partial [slices][rows][2 dim]
+int prompt_swiglu_launch(const float * partial, int32_t slices, int32_t rows, int32_t dim, uint16_t * Xf,
+                         hipStream_t stream);
+int prompt_sum_launch(const float * partial, int32_t slices, int32_t rows, int32_t dim, float * y, hipStream_t stream);
 // Prefill GEMM on bf16-exact weights over the three-part split input (gemm_split3.hip):
 // Y[M][N] (+)= sum_p Xs[M][p K .. p K + K) W16[N][K]^T, f32 products and sums; with act != nullptr (Y null,
 // no accumulate) W16 = [gate rows; up rows] (2 N rows) and act[M][3 N] = split of silu(gate) * up.
@@ -67,15 +93,17 @@ struct StepTail {
 };
 int argmax_launch(const float * logits, int32_t rows, int32_t vocab, int32_t * ids, void * workspace,
                   hipStream_t stream, const StepTail & tail = StepTail{});
-// split (optional): write the rows as the three-part bf16 split of the prefill GEMM's input ([rows][3 dim],
-// see split_bf16x3_rows_launch) instead of f32 rows of y / a
 int rmsnorm_rows_launch(const float * x, const float * w, int32_t rows, int32_t dim, float eps, float * y,
-                        hipStream_t stream, uint16_t * split = nullptr);
-int swiglu_rows_launch(const float * gu, int32_t rows, int32_t dim, float * a, hipStream_t stream,
-                       uint16_t * split = nullptr);
+                        hipStream_t stream);
+int swiglu_rows_launch(const float * gu, int32_t rows, int32_t dim, float * a, hipStream_t stream);
 // stats (optional, rows <= 32): [ceil(dim / 32)][32] partial sums of squares of each gathered row
 int embed_rows_launch(const float * table, int32_t n_rows, int32_t dim, const int32_t * ids, int32_t rows,
                       float * out, hipStream_t stream, double * stats = nullptr);
+// qa_kv_append of one stream's rows; slices > 0: qkv is the projection's partial sums [slices][n_tokens][q|k|v width],
+// added up in slice order
+int kv_append_launch(const float * qkv, int32_t slices, const float * q_norm_w, const float * k_norm_w, float * q_out,
+                     void * cache, const qa_kv_layout & layout, int32_t layer, const int32_t * n_past, int32_t n_streams,
+                     int32_t n_tokens, int32_t n_heads, float rope_theta, float eps, hipStream_t stream);
 int advance_lens_launch(int32_t * lens, int32_t n, int32_t delta, hipStream_t stream);
 int set_values_launch(int32_t * dst, int32_t n, int32_t value, hipStream_t stream);
 int cast_rows_launch(const float * src, void * dst, int32_t cache_type, int64_t n, hipStream_t stream);
