@@ -194,36 +194,40 @@ __global__ __launch_bounds__(256) void prefill_rows_kernel(RowsParams p) {
         (red[0][hh][d] + red[1][hh][d]) + (red[2][hh][d] + red[3][hh][d]);
 }
 
-// f32 K/V on f32 MFMA (v_mfma_f32_16x16x4_f32: exact f32 products, f32 sums).  A workgroup owns 64
-// queries x both query heads of one KV head (8 waves: wave w takes head w % 2 and queries 16 (w / 2) ..
-// + 15) and walks the keys in tiles of 32, staged in LDS (double-buffered, the next tile in registers
-// while the current one is computed).  Each wave computes S^T = K Q^T (keys x queries): the operand
-// layout of the product then holds, in each lane, 4 keys of one query, which is exactly the B operand
-// of O^T = V^T P^T, so P never moves.  Softmax is online, in f32, with the running sum in double:
-// p_j = exp(s_j - m) rescaled as m grows, and o / l at the end -- the same f32 arithmetic as
+// f32 K/V on f32 MFMA (v_mfma_f32_16x16x4_f32: exact f32 products, f32 sums).  A workgroup of 8 waves owns 64 / KG
+// queries x both query heads of one KV head; KG key groups of waves walk the causal key tiles (32 keys) in turn, group
+// g the tiles g, g + KG, ..., each staged in LDS (the next tile in registers while the current one is computed), and
+// the groups' online-softmax states are merged through LDS at the end, in group order.  Each wave computes
+// S^T = K Q^T (keys x queries) for 16 queries of one head: the operand layout of the product then holds, in each lane, 4
+// keys of one query, which is exactly the B operand of O^T = V^T P^T, so P never moves.  Softmax is online, in f32, with
+// the running sum in double: p_j = exp(s_j - m) rescaled as m grows, and o / l at the end -- the same f32 arithmetic as
 // prefill_rows_kernel in another association (about 1e-6 relative).
 // Lane layouts of v_mfma_f32_16x16x4_f32 (lane l, g = l / 16): A[m = l % 16][k = g], B[k = g][n = l % 16],
 // C[m = 4 g + i][n = l % 16], i = 0..3.
 constexpr int kF32Tile = 32;                  // keys per tile
 constexpr int kF32KLs = kHeadDim + 8;         // K row stride in LDS (floats): 16-byte reads of 16 rows
 constexpr int kF32VLs = kHeadDim + 16;        // V row stride: the 4 lane groups read 4 rows of one column
-constexpr int kF32Queries = 64;
+constexpr int kF32Stage = kF32Tile * (kF32KLs + kF32VLs);   // floats of one staged tile: K, then V
 
 typedef float f4v __attribute__((ext_vector_type(4)));
 
-// One query block of 64 (8 waves) against its causal key range.
-__device__ inline void f32mfma_block(const RowsParams & p, float (*ks)[kF32Tile * kF32KLs],
-                                     float (*vs)[kF32Tile * kF32VLs], int qb) {
-    const int kvh = blockIdx.y;
+// One query block (64 / KG queries) against its causal key range.  lds: KG x NBUF stages.
+template <int KG, int NBUF>
+__device__ inline void f32mfma_block(const RowsParams & p, float * lds, int kvh, int qb) {
+    constexpr int kQueries = 64 / KG;
+    constexpr int kGroupThreads = 512 / KG;
+    constexpr int kLoads = kF32Tile * 32 / kGroupThreads;     // 16-byte loads per thread and array
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x >> 6;
+    const int kg = wave / (8 / KG), gw = wave % (8 / KG);
     const int g = lane >> 4, c = lane & 15;
-    const int hh = wave & 1, qi = wave >> 1;
-    const int q0 = qb * kF32Queries;
+    const int hh = gw & 1, qi = gw >> 1;
+    const int q0 = qb * kQueries;
     const int qrow = q0 + 16 * qi + c;                              // this lane's query (token index)
     const int qpos = p.n_past + min(qrow, p.n_tokens - 1);          // its position (rows past T: the last)
-    const int n_keys = p.n_past + min(q0 + kF32Queries, p.n_tokens);   // keys of the workgroup's last query
+    const int n_keys = p.n_past + min(q0 + kQueries, p.n_tokens);   // keys of the workgroup's last query
     const int n_tiles = (n_keys + kF32Tile - 1) / kF32Tile;
+    const int steps = (n_tiles + KG - 1) / KG;                      // the same for every group
 
     // q of this lane's query, d = 16 u + 4 g + 0..3 (the B operand order)
     f4v qreg[8];
@@ -235,27 +239,35 @@ __device__ inline void f32mfma_block(const RowsParams & p, float (*ks)[kF32Tile 
     }
     const float * kbase = static_cast<const float *>(p.k) + kvh * p.head_stride;
     const float * vbase = static_cast<const float *>(p.v) + kvh * p.head_stride;
-    // tile staging: thread t loads 16 bytes at key t / 32 (+ 16), d 4 (t % 32), for K and for V
-    const int lk = threadIdx.x >> 5, ld = 4 * (threadIdx.x & 31);
-    f4v kr[2], vr[2];
-    auto load_tile = [&](int tile) {
+    float * stage0 = lds + kg * NBUF * kF32Stage;
+    // tile staging: thread t of the group loads 16 bytes at key t / 32 (+ kGroupThreads / 32), d 4 (t % 32)
+    const int gt = threadIdx.x % kGroupThreads;
+    const int lk = gt >> 5, ld = 4 * (gt & 31);
+    f4v kr[kLoads], vr[kLoads];
+    auto load_tile = [&](int step) {
+        const int tile = step * KG + kg;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int key = min(tile * kF32Tile + lk + 16 * h, n_keys - 1);
+        for (int h = 0; h < kLoads; ++h) {
+            const int key = min(tile * kF32Tile + lk + kGroupThreads / 32 * h, n_keys - 1);
             kr[h] = *reinterpret_cast<const f4v *>(kbase + static_cast<int64_t>(key) * p.row_stride + ld);
             vr[h] = *reinterpret_cast<const f4v *>(vbase + static_cast<int64_t>(key) * p.row_stride + ld);
         }
     };
     auto store_tile = [&](int buf) {
+        float * st = stage0 + buf * kF32Stage;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            *reinterpret_cast<f4v *>(&ks[buf][(lk + 16 * h) * kF32KLs + ld]) = kr[h];
-            *reinterpret_cast<f4v *>(&vs[buf][(lk + 16 * h) * kF32VLs + ld]) = vr[h];
+        for (int h = 0; h < kLoads; ++h) {
+            *reinterpret_cast<f4v *>(st + (lk + kGroupThreads / 32 * h) * kF32KLs + ld) = kr[h];
+            *reinterpret_cast<f4v *>(st + kF32Tile * kF32KLs + (lk + kGroupThreads / 32 * h) * kF32VLs + ld) = vr[h];
         }
     };
     load_tile(0);
+    // q is waited for here, with the first tile: left to the loop, its wait there would also wait for the tile loads
+    // in flight in every step
+#pragma unroll
+    for (int u = 0; u < 8; ++u) asm volatile("" : "+v"(qreg[u]));
     store_tile(0);
-    if (n_tiles > 1) load_tile(1);
+    if (steps > 1) load_tile(1);
     __syncthreads();
 
     f4v oacc[8];
@@ -263,78 +275,131 @@ __device__ inline void f32mfma_block(const RowsParams & p, float (*ks)[kF32Tile 
     for (int db = 0; db < 8; ++db) oacc[db] = f4v{0.f, 0.f, 0.f, 0.f};
     float m_run = -INFINITY;
     double l_run = 0.0;
-    for (int t = 0; t < n_tiles; ++t) {
-        const int buf = t & 1;
-        const float * kt = ks[buf];
-        const float * vt = vs[buf];
-        // S^T for keys 16 b + 0..15 of the tile
-        f4v sacc[2];
-#pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            sacc[b] = f4v{0.f, 0.f, 0.f, 0.f};
-            const float * kr_l = kt + (16 * b + c) * kF32KLs + 4 * g;
+    for (int t = 0; t < steps; ++t) {
+        const int buf = NBUF == 2 ? t & 1 : 0;
+        const int tile = t * KG + kg;
+        if (tile < n_tiles) {
+            const float * kt = stage0 + buf * kF32Stage;
+            const float * vt = kt + kF32Tile * kF32KLs;
+            // S^T for keys 16 b + 0..15 of the tile (the two blocks' MFMA chains alternate)
+            f4v sacc[2] = {f4v{0.f, 0.f, 0.f, 0.f}, f4v{0.f, 0.f, 0.f, 0.f}};
+            const float * kr_l = kt + c * kF32KLs + 4 * g;
+            f4v a[2][2];
+            auto read_k = [&](int u) {
+                a[u & 1][0] = *reinterpret_cast<const f4v *>(kr_l + 16 * u);
+                a[u & 1][1] = *reinterpret_cast<const f4v *>(kr_l + 16 * kF32KLs + 16 * u);
+            };
+            read_k(0);
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
-                const f4v a = *reinterpret_cast<const f4v *>(kr_l + 16 * u);
+                if (u < 7) read_k(u + 1);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) sacc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], qreg[u][j], sacc[b], 0, 0, 0);
+                for (int j = 0; j < 4; ++j) {
+                    sacc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u & 1][0][j], qreg[u][j], sacc[0], 0, 0, 0);
+                    sacc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u & 1][1][j], qreg[u][j], sacc[1], 0, 0, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
             }
-        }
-        // scale, causal mask, online softmax of this lane's query over the tile's 32 keys
-        float sv[2][4];
-        float mx = -INFINITY;
+            // scale, causal mask, online softmax of this lane's query over the tile's 32 keys
+            float sv[2][4];
+            float mx = -INFINITY;
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
+            for (int b = 0; b < 2; ++b) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int kp = t * kF32Tile + 16 * b + 4 * g + i;
-                const float x = kp <= qpos ? sacc[b][i] * p.scale : -INFINITY;
-                sv[b][i] = x;
-                mx = fmaxf(mx, x);
-            }
-        }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
-        const float m_new = fmaxf(m_run, mx);
-        const float corr = m_run == -INFINITY ? 0.0f : expf(m_run - m_new);
-        float psum = 0.0f;
-#pragma unroll
-        for (int b = 0; b < 2; ++b) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float e = sv[b][i] == -INFINITY ? 0.0f : expf(sv[b][i] - m_new);
-                sv[b][i] = e;
-                psum += e;
-            }
-        }
-        psum += __shfl_xor(psum, 16, kWave);
-        psum += __shfl_xor(psum, 32, kWave);
-        l_run = l_run * static_cast<double>(corr) + static_cast<double>(psum);
-        m_run = m_new;
-#pragma unroll
-        for (int db = 0; db < 8; ++db) oacc[db] *= corr;
-        // O^T[d][q] += V^T[d][key] P^T[key][q]: keys 16 b + 4 g + i of the tile in k-slot g of step (b, i)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float * vrow = vt + (16 * b + 4 * g + i) * kF32VLs + c;
-#pragma unroll
-                for (int db = 0; db < 8; ++db) {
-                    oacc[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(vrow[16 * db], sv[b][i], oacc[db], 0, 0, 0);
+                for (int i = 0; i < 4; ++i) {
+                    const int kp = tile * kF32Tile + 16 * b + 4 * g + i;
+                    const float x = kp <= qpos ? sacc[b][i] * p.scale : -INFINITY;
+                    sv[b][i] = x;
+                    mx = fmaxf(mx, x);
                 }
             }
+            mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
+            mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+            const float m_new = fmaxf(m_run, mx);
+            const float corr = m_run == -INFINITY ? 0.0f : expf(m_run - m_new);
+            float psum = 0.0f;
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float e = sv[b][i] == -INFINITY ? 0.0f : expf(sv[b][i] - m_new);
+                    sv[b][i] = e;
+                    psum += e;
+                }
+            }
+            psum += __shfl_xor(psum, 16, kWave);
+            psum += __shfl_xor(psum, 32, kWave);
+            l_run = l_run * static_cast<double>(corr) + static_cast<double>(psum);
+            m_run = m_new;
+#pragma unroll
+            for (int db = 0; db < 8; ++db) oacc[db] *= corr;
+            // O^T[d][q] += V^T[d][key] P^T[key][q]: keys 16 b + 4 g + i of the tile in k-slot g of step 4 b + i; the
+            // next step's V values are read from LDS before a step's MFMAs
+            float vv[2][8];
+            auto read_v = [&](int st) {
+                const float * vrow = vt + (16 * (st >> 2) + 4 * g + (st & 3)) * kF32VLs + c;
+#pragma unroll
+                for (int db = 0; db < 8; ++db) vv[st & 1][db] = vrow[16 * db];
+            };
+            read_v(0);
+#pragma unroll
+            for (int st = 0; st < 8; ++st) {
+                if (st < 7) read_v(st + 1);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int db = 0; db < 8; ++db) {
+                    oacc[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[st & 1][db], sv[st >> 2][st & 3], oacc[db], 0, 0, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
-        // stage the next tile (its loads were issued a tile ago) and issue the loads of the one after.
-        // Buffer buf ^ 1 last held tile t - 1, which every wave finished before the previous barrier.
-        if (t + 1 < n_tiles) {
-            store_tile(buf ^ 1);
-            if (t + 2 < n_tiles) load_tile(t + 2);
+        // stage the next tile (its loads were issued a tile ago) and issue the loads of the one after.  Two buffers:
+        // buf ^ 1 last held the tile before, which every wave finished before the previous barrier.
+        if (t + 1 < steps) {
+            if (NBUF == 1) __syncthreads();
+            store_tile(NBUF == 2 ? buf ^ 1 : 0);
+            if (t + 2 < steps) load_tile(t + 2);
             __syncthreads();
         }
     }
+    if constexpr (KG > 1) {
+        // merge: groups 1 .. KG - 1 leave O, m and l of their waves in LDS, group 0 adds them in order
+        __syncthreads();
+        constexpr int kWaves = 8 / KG;                               // waves of a group
+        float * so = lds;                                            // [(KG - 1) kWaves][32][64]
+        double * sl = reinterpret_cast<double *>(so + (KG - 1) * kWaves * 32 * kWave);
+        float * sm = reinterpret_cast<float *>(sl + (KG - 1) * kWaves * kWave);
+        if (kg > 0) {
+            const int w = (kg - 1) * kWaves + gw;
+#pragma unroll
+            for (int db = 0; db < 8; ++db)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) so[(w * 32 + db * 4 + i) * kWave + lane] = oacc[db][i];
+            sl[w * kWave + lane] = l_run;
+            sm[w * kWave + lane] = m_run;
+        }
+        __syncthreads();
+        if (kg == 0) {
+            for (int o = 1; o < KG; ++o) {
+                const int w = (o - 1) * kWaves + gw;
+                const float mo = sm[w * kWave + lane];
+                if (mo == -INFINITY) continue;                       // no key of the group before this query
+                const float m_new = fmaxf(m_run, mo);
+                const float ca = expf(m_run - m_new), cb = expf(mo - m_new);
+                l_run = l_run * static_cast<double>(ca) + sl[w * kWave + lane] * static_cast<double>(cb);
+                m_run = m_new;
+#pragma unroll
+                for (int db = 0; db < 8; ++db)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        oacc[db][i] = oacc[db][i] * ca + so[(w * 32 + db * 4 + i) * kWave + lane] * cb;
+                    }
+            }
+        }
+    }
     // oacc[db][i] = O^T[d = 16 db + 4 g + i][q = c]; normalise and store
-    if (qrow < p.n_tokens) {
+    if (kg == 0 && qrow < p.n_tokens) {
         const float r = static_cast<float>(1.0 / l_run);
         float * out = p.out + static_cast<int64_t>(qrow) * p.out_stride + (kRep * kvh + hh) * kHeadDim + 4 * g;
 #pragma unroll
@@ -345,27 +410,41 @@ __device__ inline void f32mfma_block(const RowsParams & p, float (*ks)[kF32Tile 
     }
 }
 
-__global__ __launch_bounds__(512) void prefill_f32mfma_kernel(RowsParams p) {
-    __shared__ __attribute__((aligned(16))) float ks[2][kF32Tile * kF32KLs];
-    __shared__ __attribute__((aligned(16))) float vs[2][kF32Tile * kF32VLs];
-    const int n_qb = (p.n_tokens + kF32Queries - 1) / kF32Queries;
-    // causal balance: workgroup i takes query block n_qb - 1 - i, then block i, so every workgroup
-    // walks about the same number of key tiles
-    const int first = n_qb - 1 - static_cast<int>(blockIdx.x);
-    f32mfma_block(p, ks, vs, first);
-    const int second = static_cast<int>(blockIdx.x);
-    if (second < first) {
-        __syncthreads();                 // every wave is done with the first block's LDS tiles
-        f32mfma_block(p, ks, vs, second);
-    }
+// Workgroup i serves KV head i % n_kv (one head per XCD for 8 heads, whose K and V stay in that L2) and query block
+// n_qb - 1 - i / n_kv: longest first, so that the short blocks fill the CUs behind them.
+template <int KG, int NBUF>
+__global__ __launch_bounds__(512) void prefill_f32mfma_kernel(RowsParams p, int n_kv) {
+    extern __shared__ __attribute__((aligned(16))) float lds_f32[];
+    const int n_qb = (p.n_tokens + 64 / KG - 1) / (64 / KG);
+    f32mfma_block<KG, NBUF>(p, lds_f32, static_cast<int>(blockIdx.x) % n_kv,
+                            n_qb - 1 - static_cast<int>(blockIdx.x) / n_kv);
 }
 
-int launch_f32mfma(const RowsParams & p, int n_kv_heads, hipStream_t stream) {
-    const int n_qb = (p.n_tokens + kF32Queries - 1) / kF32Queries;
-    hipLaunchKernelGGL(prefill_f32mfma_kernel, dim3(static_cast<unsigned>((n_qb + 1) / 2), static_cast<unsigned>(n_kv_heads)),
-                       dim3(512), 0, stream, p);
+template <int KG, int NBUF>
+int launch_f32_groups(const RowsParams & p, int n_kv_heads, hipStream_t stream) {
+    const int n_qb = (p.n_tokens + 64 / KG - 1) / (64 / KG);
+    const size_t merge = KG > 1 ? static_cast<size_t>(KG - 1) * (8 / KG) * kWave * (32 * 4 + 8 + 4) : 0;
+    const size_t lds = std::max(sizeof(float) * KG * NBUF * kF32Stage, merge);
+    QA_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(prefill_f32mfma_kernel<KG, NBUF>),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+    hipLaunchKernelGGL((prefill_f32mfma_kernel<KG, NBUF>), dim3(static_cast<unsigned>(n_qb * n_kv_heads)), dim3(512), lds,
+                       stream, p, n_kv_heads);
     QA_LAUNCH_CHECK("prefill_f32mfma_kernel");
     return QA_OK;
+}
+
+// Key groups by the number of workgroups.  A CU holds one workgroup (LDS, or registers), and a step of 32 keys per group
+// takes about 5 us whatever the split, so short prompts gain from more, shorter workgroups: with one group 1037 tokens
+// made 72 workgroups (paired for balance) of 36 steps, 193 us; four groups make 520 of at most 9, 79 us.  Many
+// workgroups pay for their start, the merge and the K/V tiles that more blocks re-read, so the groups go down as the
+// grid grows past about 2.5 and 3.4 workgroups per CU.  us by groups 4 / 2 / 1: 156 tokens 16 / 19 / 27 (42 before), 156
+// behind 1000 63 / 102 / 180 (366), 640 37 / 58 / 101 (121), 1037 79 / 94 / 164 (193), 1500 140 / 133 / 230 (269), 2500
+// 344 / 315 / 385 (441), 3000 455 / 431 / 464 (520), 3913 774 / 661 / 642 (690).
+int launch_f32mfma(const RowsParams & p, int n_kv_heads, hipStream_t stream) {
+    auto workgroups = [&](int queries) { return (p.n_tokens + queries - 1) / queries * n_kv_heads; };
+    if (workgroups(16) <= 640) return launch_f32_groups<4, 1>(p, n_kv_heads, stream);
+    if (workgroups(32) <= 864) return launch_f32_groups<2, 2>(p, n_kv_heads, stream);
+    return launch_f32_groups<1, 2>(p, n_kv_heads, stream);
 }
 
 // QA_PREFILL_F32_ROWS=1 keeps the f32 row kernel (comparison)
