@@ -359,7 +359,8 @@ int run_layer(qa_decoder * d, int32_t l, int32_t rows, int kind, int32_t n_past,
     const int32_t W3 = QD + 2 * KD;
     hipStream_t s = d->stream;
     const bool prompt = rows > 1 && !fused && d->xf;
-    int32_t slices = 0;   // K slices of the q|k|v projection, still partial sums in d->partial
+    int32_t slices = 0;        // K slices of the q|k|v projection, still partial sums in d->partial
+    bool attn_split = false;   // the attention left its output split in d->xf
     int rc;
     {
         Prof pr(d, kFamProj);
@@ -390,7 +391,7 @@ int run_layer(qa_decoder * d, int32_t l, int32_t rows, int kind, int32_t n_past,
         }
         Prof pr(d, kFamPrefillAttn);
         rc = causal_f32_launch(d->qkv, W3, d->qkv + QD, d->qkv + QD + KD, W3, rows, c.n_heads, c.n_kv_heads,
-                               d->scale, d->attn, QD, s);
+                               d->scale, d->attn, QD, prompt ? d->xf : nullptr, &attn_split, s);
         if (rc != QA_OK) return rc;
     } else if (kind == kDecode) {
         // append + attend in one launch: one token per stream at position d_lens[s]
@@ -408,13 +409,13 @@ int run_layer(qa_decoder * d, int32_t l, int32_t rows, int kind, int32_t n_past,
         }
         Prof pr(d, kFamPrefillAttn);
         rc = prefill_attn_launch(d->qrot, QD, d->cache, d->layout, l, 0, n_past, rows, c.n_heads, d->scale,
-                                 d->attn, d->pf_ws, d->pf_ws_bytes, s);
+                                 d->attn, prompt ? d->xf : nullptr, &attn_split, d->pf_ws, d->pf_ws_bytes, s);
         if (rc != QA_OK) return rc;
     }
     Prof pr(d, kFamProj);
     if (prompt) {
         int32_t po = 0, pg = 0;
-        rc = prompt_split_launch(d->attn, rows, QD, d->xf, s);
+        if (!attn_split) rc = prompt_split_launch(d->attn, rows, QD, d->xf, s);
         if (rc == QA_OK) rc = prompt_gemm(d, L.o16, L.o3, H, QD, d->xf, rows, d->x, true, nullptr, &po);
         if (rc == QA_OK) rc = prompt_norm_launch(d->x, d->partial, po, L.ffn_norm, rows, H, c.rms_norm_eps, d->xf, s);
         if (rc == QA_OK) rc = prompt_gemm(d, L.gu16, L.gu3, I, H, d->xf, rows, nullptr, false, d->actf, &pg);

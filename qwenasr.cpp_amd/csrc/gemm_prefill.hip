@@ -258,23 +258,16 @@ __global__ __launch_bounds__(64 * kMaxWaves) void gemm_prefill_kernel(PgParams p
         const int n16 = p.N / 16;
 #pragma unroll
         for (int q = 0; q < NT / 2; ++q) {
-            const int c16 = (ng * (kCols / 2) + 32 * q) / 16;
+            const int c = ng * (kCols / 2) + 32 * q;
 #pragma unroll
             for (int o = 0; o < 4; ++o) {
-                uint16_t part[3][4];
+                float v[4];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const float g = acc[2 * q][4 * o + e], u = acc[2 * q + 1][4 * o + e];
-                    split3_parts((g / (1.0f + expf(-g))) * u, part[0][e], part[1][e], part[2][e]);
+                    v[e] = (g / (1.0f + expf(-g))) * u;
                 }
-                uint16_t * d = p.act + (static_cast<int64_t>(mtc) * n16 + c16 + (o >> 1)) * 3 * 512 +
-                               (rr + 32 * (o & 1)) * 8 + 4 * h;
-#pragma unroll
-                for (int w = 0; w < 3; ++w) {
-                    *reinterpret_cast<uint2 *>(d + w * 512) =
-                        make_uint2(part[w][0] | (static_cast<uint32_t>(part[w][1]) << 16),
-                                   part[w][2] | (static_cast<uint32_t>(part[w][3]) << 16));
-                }
+                store_frag4(p.act, n16, 32 * mtc + rr, c + 8 * o + 4 * h, v[0], v[1], v[2], v[3]);
             }
         }
     } else {

@@ -164,15 +164,19 @@ struct PersistLaunch {
 };
 int persist_layers_launch(const PersistLaunch & a, hipStream_t stream);
 
+// split (optional): the outputs go there as the fragment-ordered split input of the o projection instead of to out;
+// *did_split says whether they did (the f32 row kernel and the two-pass f16 kernels write out only)
 int prefill_attn_launch(const float * q, int32_t q_stride, const void * cache, const qa_kv_layout & layout,
                         int32_t layer, int32_t stream_idx, int32_t n_past, int32_t n_tokens, int32_t n_heads,
-                        float scale, float * out, void * workspace, size_t workspace_bytes, hipStream_t stream);
+                        float scale, float * out, uint16_t * split, bool * did_split, void * workspace,
+                        size_t workspace_bytes, hipStream_t stream);
+bool prefill_exact();   // QA_PREFILL_EXACT=1: f16 caches on the two-pass kernels
 size_t prefill_mfma_workspace_bytes(int32_t n_tokens, int32_t n_kv);
 int prefill_mfma_launch(const float * q, int32_t q_stride, const void * k, const void * v, int64_t head_stride,
-                        int32_t n_past, int32_t n_tokens, int32_t n_kv, float scale, float * out, void * workspace,
-                        size_t workspace_bytes, hipStream_t stream);
+                        int32_t n_past, int32_t n_tokens, int32_t n_kv, float scale, float * out, uint16_t * split,
+                        void * workspace, size_t workspace_bytes, hipStream_t stream);
 int causal_f32_launch(const float * q, int32_t q_stride, const float * k, const float * v, int64_t row_stride,
                       int32_t n_tokens, int32_t n_heads, int32_t n_kv_heads, float scale, float * out,
-                      int32_t out_stride, hipStream_t stream);
+                      int32_t out_stride, uint16_t * split, bool * did_split, hipStream_t stream);
 
 }  // namespace qa

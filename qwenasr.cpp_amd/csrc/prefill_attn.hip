@@ -14,6 +14,7 @@
 // f32 throughout: one workgroup per (query, KV head), both query heads of the GQA group share every
 // loaded K/V element, the scores of the query stay in LDS (keys <= 8192).
 #include "ops.hpp"
+#include "split3.hpp"
 
 #include <cmath>
 #include <cstdlib>
@@ -35,6 +36,8 @@ struct RowsParams {
     int32_t out_stride;       // elements between the output rows of two tokens
     int32_t n_past, n_tokens;
     float scale;
+    uint16_t * split;         // prefill_f32mfma_kernel: when set, the outputs go here as the split input of a GEMM
+    int32_t split_k16;        // its row width / 16
 };
 
 template <typename CT>
@@ -401,11 +404,13 @@ __device__ inline void f32mfma_block(const RowsParams & p, float * lds, int kvh,
     // oacc[db][i] = O^T[d = 16 db + 4 g + i][q = c]; normalise and store
     if (kg == 0 && qrow < p.n_tokens) {
         const float r = static_cast<float>(1.0 / l_run);
-        float * out = p.out + static_cast<int64_t>(qrow) * p.out_stride + (kRep * kvh + hh) * kHeadDim + 4 * g;
+        const int col = (kRep * kvh + hh) * kHeadDim + 4 * g;
+        float * out = p.out + static_cast<int64_t>(qrow) * p.out_stride + col;
 #pragma unroll
         for (int db = 0; db < 8; ++db) {
             f4v o = oacc[db] * r;
-            *reinterpret_cast<f4v *>(out + 16 * db) = o;
+            if (p.split) store_frag4(p.split, p.split_k16, qrow, col + 16 * db, o[0], o[1], o[2], o[3]);
+            else *reinterpret_cast<f4v *>(out + 16 * db) = o;
         }
     }
 }
@@ -467,7 +472,9 @@ int launch_rows(const RowsParams & p, int n_kv_heads, hipStream_t stream) {
 
 int prefill_attn_launch(const float * q, int32_t q_stride, const void * cache, const qa_kv_layout & layout,
                         int32_t layer, int32_t stream_idx, int32_t n_past, int32_t n_tokens, int32_t n_heads,
-                        float scale, float * out, void * workspace, size_t workspace_bytes, hipStream_t stream) {
+                        float scale, float * out, uint16_t * split, bool * did_split, void * workspace,
+                        size_t workspace_bytes, hipStream_t stream) {
+    if (did_split) *did_split = split != nullptr;
     if (layout.head_dim != kHeadDim || n_heads != kRep * layout.n_kv_heads) {
         return fail(QA_ERR_INVALID, "prefill attention: only head_dim 128 with 2 query heads per KV head");
     }
@@ -482,8 +489,10 @@ int prefill_attn_launch(const float * q, int32_t q_stride, const void * cache, c
     const void * v0 = base + esz * cache_row_offset(layer, 1, stream_idx, 0, 0, layout.n_streams, layout.n_kv_heads,
                                                     layout.max_seq);
     if (layout.cache_type == QA_CACHE_F16) {
+        if (prefill_exact()) split = nullptr;      // the two-pass kernels write out only
+        if (did_split) *did_split = split != nullptr;
         return prefill_mfma_launch(q, q_stride, k0, v0, static_cast<int64_t>(layout.max_seq) * kHeadDim, n_past,
-                                   n_tokens, layout.n_kv_heads, scale, out, workspace, workspace_bytes, stream);
+                                   n_tokens, layout.n_kv_heads, scale, out, split, workspace, workspace_bytes, stream);
     }
     if (n_past + n_tokens > kMaxRowsKeys) {
         return fail(QA_ERR_INVALID, "prefill attention: more than 8192 keys with an f32 cache");
@@ -500,7 +509,10 @@ int prefill_attn_launch(const float * q, int32_t q_stride, const void * cache, c
     p.row_stride = kHeadDim;
     p.k = k0;
     p.v = v0;
+    p.split = split;
+    p.split_k16 = n_heads * kHeadDim / 16;
     if (!f32_rows_forced()) return launch_f32mfma(p, layout.n_kv_heads, stream);
+    if (did_split) *did_split = false;
     return launch_rows<float, false>(p, layout.n_kv_heads, stream);
 }
 
@@ -517,14 +529,15 @@ extern "C" int qa_prefill_attn(const float * q, const void * cache, const qa_kv_
     if (qa_kv_layout_check(layout) != QA_OK) return QA_ERR_INVALID;
     if (!q || !cache || !out) return fail(QA_ERR_INVALID, "qa_prefill_attn: null pointer");
     return prefill_attn_launch(q, n_heads * kHeadDim, cache, *layout, layer, stream_idx, n_past, n_tokens, n_heads,
-                               scale, out, workspace, workspace_bytes, as_stream(stream));
+                               scale, out, nullptr, nullptr, workspace, workspace_bytes, as_stream(stream));
 }
 
 namespace qa {
 
 int causal_f32_launch(const float * q, int32_t q_stride, const float * k, const float * v, int64_t row_stride,
                       int32_t n_tokens, int32_t n_heads, int32_t n_kv_heads, float scale, float * out,
-                      int32_t out_stride, hipStream_t stream) {
+                      int32_t out_stride, uint16_t * split, bool * did_split, hipStream_t stream) {
+    if (did_split) *did_split = split != nullptr;
     if (!q || !k || !v || !out || n_tokens <= 0 || n_kv_heads <= 0 || n_heads != kRep * n_kv_heads) {
         return fail(QA_ERR_INVALID, "causal f32 attention: invalid arguments");
     }
@@ -546,7 +559,10 @@ int causal_f32_launch(const float * q, int32_t q_stride, const float * k, const 
     p.scale = scale;
     p.head_stride = kHeadDim;
     p.row_stride = row_stride;
+    p.split = split;
+    p.split_k16 = n_heads * kHeadDim / 16;
     if (!f32_rows_forced()) return launch_f32mfma(p, n_kv_heads, stream);
+    if (did_split) *did_split = false;
     return launch_rows<float, false>(p, n_kv_heads, stream);
 }
 
@@ -555,6 +571,6 @@ int causal_f32_launch(const float * q, int32_t q_stride, const float * k, const 
 extern "C" int qa_causal_attn_f32(const float * q, const float * k, const float * v, int32_t n_tokens,
                                   int32_t n_heads, int32_t n_kv_heads, float scale, float * out, void * stream) {
     return qa::causal_f32_launch(q, n_heads * qa::kHeadDim, k, v, static_cast<int64_t>(n_kv_heads) * qa::kHeadDim,
-                                 n_tokens, n_heads, n_kv_heads, scale, out, n_heads * qa::kHeadDim,
+                                 n_tokens, n_heads, n_kv_heads, scale, out, n_heads * qa::kHeadDim, nullptr, nullptr,
                                  qa::as_stream(stream));
 }

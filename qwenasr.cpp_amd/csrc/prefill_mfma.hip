@@ -40,6 +40,7 @@
 // uncut tile) of one KV head is a work item, pulled from that head's queue by the workgroups serving
 // the head, longest first (see the work plan below).
 #include "ops.hpp"
+#include "split3.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -95,6 +96,7 @@ struct MfmaParams {
     const _Float16 * k;       // this layer/stream's K rows, head 0 position 0
     const _Float16 * v;
     float * out;              // [T][q_stride]
+    uint16_t * split;         // SPLIT kernels: the outputs go here instead, as the split input of the o projection
     int64_t head_stride;      // elements between KV heads (max_seq * 128)
     int32_t q_stride;
     int32_t n_past, n_tokens, n_kv, n_qt;
@@ -403,12 +405,19 @@ __device__ inline Item item_of(const MfmaParams & p, int g, int k) {
     return it;
 }
 
+// 4 consecutive outputs of token t, from column col on (SPLIT: as the split input of the o projection)
+template <bool SPLIT>
+__device__ inline void store_out(const MfmaParams & p, int t, int col, f4 v) {
+    if constexpr (SPLIT) store_frag4(p.split, p.n_kv * 2 * kHeadDim / 16, t, col, v[0], v[1], v[2], v[3]);
+    else *reinterpret_cast<f4 *>(p.out + static_cast<int64_t>(t) * p.q_stride + col) = v;
+}
+
 // One work item.  PASS 1: the part's row statistics (max and sum of exp) of its kCols query columns.
 // PASS 2: p over the part's keys with the statistics of both parts of its query tile, and
 // O^T += V^T P^T; the two parts of a cut tile are added by whichever finishes second.
 // PASS 3 (single pass): online softmax over the part's keys (online_tile); the part's O, max and sum are
 // combined with the other part's by whichever finishes second, then O / sum is stored.
-template <int PASS>
+template <int PASS, bool SPLIT>
 __device__ inline void run_item(const MfmaParams & p, const Item & it, _Float16 (*sK)[kBK * kKS],
                                 _Float16 (*sV)[kHeadDim * kVS]) {
     constexpr bool kWithV = PASS != 1;
@@ -635,13 +644,243 @@ __device__ inline void run_item(const MfmaParams & p, const Item & it, _Float16 
 #pragma unroll
     for (int qb = 0; qb < kQB; ++qb) {
         if (tq[qb] < p.n_tokens) {
-            float * op = p.out + static_cast<int64_t>(tq[qb]) * p.q_stride + h * kHeadDim + g4 * 4;
 #pragma unroll
-            for (int db = 0; db < 8; ++db) {
-                *reinterpret_cast<float4 *>(op + db * 16) =
-                    make_float4(O[qb][db][0], O[qb][db][1], O[qb][db][2], O[qb][db][3]);
+            for (int db = 0; db < 8; ++db) store_out<SPLIT>(p, tq[qb], h * kHeadDim + db * 16 + g4 * 4, O[qb][db]);
+        }
+    }
+}
+
+// ---------------------------------------------------------------- short prompts: key groups
+// One workgroup per 32 query tokens and KV head; wave = head (2) x key group (4).  The groups walk the causal key
+// tiles (32 keys) in turn, group kg the tiles kg, kg + 4, ..., each staged in LDS by its two waves, with the online
+// softmax of the single pass; at the end the four states of a head are merged through LDS, in group order, every wave
+// taking a quarter of the dims.  No queue, no cut tiles, no workspace.
+// What it is for: up to about 2000 tokens the 128-token tiles above are few (16 at 156 tokens) and each walks its key
+// tiles in sequence, 3.4 us a tile of 64 keys, with a merge of cut tiles across workgroups behind it.
+constexpr int kGTok = 32;                        // query tokens per workgroup
+constexpr int kGKeys = 32;                       // keys per tile
+constexpr int kGVS = 48;                         // V^T row stride (halfs): 24 dwords, conflict-free like kVS
+constexpr int kGroups = 4;
+constexpr int kGStage = kGKeys * kKS + kHeadDim * kGVS;          // halfs of one staged tile
+constexpr int kGMergeFloats = 8 * 64 * kWave;                    // every wave's O: 64 floats per lane
+constexpr size_t kGMergeBytes = (kGMergeFloats + 8 * kQB * kWave) * sizeof(float) + 8 * kQB * kWave * sizeof(double);
+constexpr size_t kGLds = std::max(kGroups * kGStage * sizeof(_Float16), kGMergeBytes);
+
+template <bool SPLIT>
+__global__ __launch_bounds__(kPfThreads, 2) void prefill_groups_kernel(MfmaParams p) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds_g[];
+    const int g = static_cast<int>(blockIdx.x) % p.n_kv;
+    const int n_qt = (p.n_tokens + kGTok - 1) / kGTok;
+    const int t0 = (n_qt - 1 - static_cast<int>(blockIdx.x) / p.n_kv) * kGTok;     // longest first
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+    const int hh = wave & 1, kg = wave >> 1;
+    const int h = g * 2 + hh;
+    const int c16 = lane & 15, g4 = lane >> 4;
+    const int kend = p.n_past + min(t0 + kGTok, p.n_tokens);
+    const int n_kt = (kend + kGKeys - 1) / kGKeys;
+    const int steps = (n_kt + kGroups - 1) / kGroups;                // the same for every group
+    const int kt_full = (p.n_past + t0 + 1) / kGKeys;                // tiles below are attended by every query
+    const _Float16 * kh = p.k + g * p.head_stride;
+    const _Float16 * vh = p.v + g * p.head_stride;
+    const float c = p.scale * kLog2e;
+    _Float16 * sK = reinterpret_cast<_Float16 *>(lds_g) + kg * kGStage;
+    _Float16 * sV = sK + kGKeys * kKS;
+
+    // staging by the group's 128 threads: K row gt / 16 + 8 i, 16-byte slice gt % 16; V keys 2 kp, 2 kp + 1 (kp = gt % 16)
+    // of dims 8 dg .. + 7 (dg = gt / 16 + 8 i), written transposed.  Rows past the end re-read the last row.
+    const int gt = hh * kWave + lane;
+    u4 rk[4], rv[2][2];
+    auto load = [&](int step) {
+        const int row0 = (step * kGroups + kg) * kGKeys;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            rk[i] = *reinterpret_cast<const u4 *>(kh + static_cast<int64_t>(min(row0 + (gt >> 4) + 8 * i, kend - 1)) * kHeadDim + (gt & 15) * 8);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                rv[i][e] = *reinterpret_cast<const u4 *>(vh + static_cast<int64_t>(min(row0 + 2 * (gt & 15) + e, kend - 1)) * kHeadDim +
+                                                         ((gt >> 4) + 8 * i) * 8);
+            }
+    };
+    auto store = [&]() {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) *reinterpret_cast<u4 *>(sK + ((gt >> 4) + 8 * i) * kKS + (gt & 15) * 8) = rk[i];
+        const int j = 2 * (gt & 15);
+        const int col = ((j & 15) >> 2) * 8 + (j >> 4) * 4 + (j & 3);            // PV order (see store_tile)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                _Float16 * d = sV + (((gt >> 4) + 8 * i) * 8 + 2 * w) * kGVS + col;
+                *reinterpret_cast<uint32_t *>(d) = lo_pair(rv[i][0][w], rv[i][1][w]);
+                *reinterpret_cast<uint32_t *>(d + kGVS) = hi_pair(rv[i][0][w], rv[i][1][w]);
+            }
+    };
+    load(0);
+
+    int tq[kQB], lim[kQB];
+    h8 qf[kQB][4];
+#pragma unroll
+    for (int qb = 0; qb < kQB; ++qb) {
+        tq[qb] = t0 + qb * 16 + c16;
+        lim[qb] = tq[qb] < p.n_tokens ? p.n_past + tq[qb] : -1;
+        const bool ok = tq[qb] < p.n_tokens;
+        const float * qp = p.q + static_cast<int64_t>(min(tq[qb], p.n_tokens - 1)) * p.q_stride + h * kHeadDim + g4 * 8;
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+            const f4 a = *reinterpret_cast<const f4 *>(qp + ks * 32), b = *reinterpret_cast<const f4 *>(qp + ks * 32 + 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                qf[qb][ks][e] = static_cast<_Float16>(ok ? a[e] : 0.f);
+                qf[qb][ks][4 + e] = static_cast<_Float16>(ok ? b[e] : 0.f);
             }
         }
+    }
+    float m[kQB];
+    double l[kQB];
+    f4 O[kQB][8];
+#pragma unroll
+    for (int qb = 0; qb < kQB; ++qb) {
+        m[qb] = -INFINITY;
+        l[qb] = 0.0;
+#pragma unroll
+        for (int db = 0; db < 8; ++db) O[qb][db] = f4{0.f, 0.f, 0.f, 0.f};
+    }
+    store();
+    if (steps > 1) load(1);
+    __syncthreads();
+    for (int s = 0; s < steps; ++s) {
+        const int kt = s * kGroups + kg;
+        if (kt < n_kt) {
+            f4 S[kQB][2];
+            h8 a[2][2];
+            auto read_k = [&](int ks) {
+#pragma unroll
+                for (int kb = 0; kb < 2; ++kb) a[ks & 1][kb] = *reinterpret_cast<const h8 *>(sK + (kb * 16 + c16) * kKS + ks * 32 + g4 * 8);
+            };
+#pragma unroll
+            for (int qb = 0; qb < kQB; ++qb)
+#pragma unroll
+                for (int kb = 0; kb < 2; ++kb) S[qb][kb] = f4{0.f, 0.f, 0.f, 0.f};
+            read_k(0);
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks) {
+                if (ks < 3) read_k(ks + 1);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                    for (int qb = 0; qb < kQB; ++qb) S[qb][kb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[ks & 1][kb], qf[qb][ks], S[qb][kb], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            h8 v[8];
+#pragma unroll
+            for (int db = 0; db < 8; ++db) v[db] = *reinterpret_cast<const h8 *>(sV + (db * 16 + c16) * kGVS + g4 * 8);
+            if (kt >= kt_full) {
+#pragma unroll
+                for (int qb = 0; qb < kQB; ++qb)
+#pragma unroll
+                    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            if (kt * kGKeys + kb * 16 + g4 * 4 + i > lim[qb]) S[qb][kb][i] = -INFINITY;
+                        }
+            }
+            // online softmax as online_tile's
+            float mn[kQB];
+            bool up[kQB];
+#pragma unroll
+            for (int qb = 0; qb < kQB; ++qb) {
+                float t = -INFINITY;
+#pragma unroll
+                for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) t = fmaxf(t, S[qb][kb][i]);
+                t = fmaxf(t, __shfl_xor(t, 16, kWave));
+                t = fmaxf(t, __shfl_xor(t, 32, kWave));
+                mn[qb] = fmaxf(m[qb], t);
+                up[qb] = (mn[qb] - m[qb]) * c > kLazyLog2;
+            }
+            if (__any(up[0] || up[1])) {
+#pragma unroll
+                for (int qb = 0; qb < kQB; ++qb) {
+                    const float f = up[qb] ? __builtin_amdgcn_exp2f((m[qb] - mn[qb]) * c) : 1.0f;
+#pragma unroll
+                    for (int db = 0; db < 8; ++db) O[qb][db] *= f;
+                    l[qb] *= static_cast<double>(f);
+                    if (up[qb]) m[qb] = mn[qb];
+                }
+            }
+            h8 pf[kQB];
+#pragma unroll
+            for (int qb = 0; qb < kQB; ++qb) {
+                const float mc = m[qb] == -INFINITY ? INFINITY : m[qb] * c;
+                float part = 0.0f;
+#pragma unroll
+                for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float e = __builtin_amdgcn_exp2f(fmaf(S[qb][kb][i], c, -mc));
+                        part += e;
+                        pf[qb][kb * 4 + i] = static_cast<_Float16>(e);
+                    }
+                l[qb] += static_cast<double>(part);
+            }
+#pragma unroll
+            for (int db = 0; db < 8; ++db)
+#pragma unroll
+                for (int qb = 0; qb < kQB; ++qb) O[qb][db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v[db], pf[qb], O[qb][db], 0, 0, 0);
+        }
+        if (s + 1 < steps) {
+            __syncthreads();                       // every wave is done with its tile
+            store();
+            if (s + 2 < steps) load(s + 2);
+            __syncthreads();
+        }
+    }
+    // merge: every wave's O, m and l (the column's sum over its 4 lanes) in LDS, then wave kg of a head takes dim blocks
+    // 2 kg and 2 kg + 1 of the four groups
+    float * so = reinterpret_cast<float *>(lds_g);
+    float * sm = so + kGMergeFloats;
+    double * sl = reinterpret_cast<double *>(sm + 8 * kQB * kWave);
+    __syncthreads();
+#pragma unroll
+    for (int qb = 0; qb < kQB; ++qb) {
+        double lt = l[qb];
+        lt += __shfl_xor(lt, 16, kWave);
+        lt += __shfl_xor(lt, 32, kWave);
+        sm[(wave * kQB + qb) * kWave + lane] = m[qb];
+        sl[(wave * kQB + qb) * kWave + lane] = lt;
+#pragma unroll
+        for (int db = 0; db < 8; ++db) *reinterpret_cast<f4 *>(so + ((wave * kQB + qb) * 8 + db) * 4 * kWave + lane * 4) = O[qb][db];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int qb = 0; qb < kQB; ++qb) {
+        if (tq[qb] >= p.n_tokens) continue;
+        float mg[kGroups], M = -INFINITY;
+#pragma unroll
+        for (int o = 0; o < kGroups; ++o) {
+            mg[o] = sm[((2 * o + hh) * kQB + qb) * kWave + lane];
+            M = fmaxf(M, mg[o]);
+        }
+        double lt = 0.0;
+        f4 out[2] = {f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int o = 0; o < kGroups; ++o) {
+            const float f = mg[o] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((mg[o] - M) * c);
+            lt += sl[((2 * o + hh) * kQB + qb) * kWave + lane] * static_cast<double>(f);
+#pragma unroll
+            for (int d = 0; d < 2; ++d) {
+                out[d] += *reinterpret_cast<const f4 *>(so + (((2 * o + hh) * kQB + qb) * 8 + 2 * kg + d) * 4 * kWave + lane * 4) * f;
+            }
+        }
+        const float r = lt > 0.0 ? static_cast<float>(1.0 / lt) : 0.0f;
+#pragma unroll
+        for (int d = 0; d < 2; ++d) store_out<SPLIT>(p, tq[qb], h * kHeadDim + (2 * kg + d) * 16 + g4 * 4, out[d] * r);
     }
 }
 
@@ -651,7 +890,7 @@ __device__ inline void run_item(const MfmaParams & p, const Item & it, _Float16 
 // head, whose K/V (2 MB at 4k positions) then stays in that XCD's L2.  Each workgroup makes exactly one
 // pull past the end of its queue; the last of those resets the counter to zero for the next call.
 // Pass 1 holds no V tile and no O: 128 registers give two workgroups per CU.
-template <int PASS>
+template <int PASS, bool SPLIT = false>
 __global__ __launch_bounds__(kPfThreads, 2) void prefill_mfma_kernel(MfmaParams p) {
     __shared__ __attribute__((aligned(16))) _Float16 sK[2][kBK * kKS];
     __shared__ __attribute__((aligned(16))) _Float16 sV[PASS != 1 ? 2 : 1][PASS != 1 ? kHeadDim * kVS : 8];
@@ -672,7 +911,7 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_mfma_kernel(MfmaParams 
             }
             return;
         }
-        run_item<PASS>(p, item_of(p, g, k), sK, reinterpret_cast<_Float16 (*)[kHeadDim * kVS]>(sV));
+        run_item<PASS, SPLIT>(p, item_of(p, g, k), sK, reinterpret_cast<_Float16 (*)[kHeadDim * kVS]>(sV));
     }
 }
 
@@ -705,6 +944,15 @@ int resident_grid() {
     return n;
 }
 
+template <bool SPLIT>
+int launch_groups(const MfmaParams & p, int64_t wgs, hipStream_t stream) {
+    QA_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(prefill_groups_kernel<SPLIT>),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kGLds)));
+    hipLaunchKernelGGL((prefill_groups_kernel<SPLIT>), dim3(static_cast<unsigned>(wgs)), dim3(kPfThreads), kGLds, stream, p);
+    QA_LAUNCH_CHECK("prefill_groups_kernel");
+    return QA_OK;
+}
+
 // Workspace: the fixed region (queue and merge counters), then the statistics of two parts per
 // (KV head, query tile), then (grids of at most kPfCutUnits units) two partial outputs per unit.
 size_t prefill_mfma_workspace_bytes(int32_t n_tokens, int32_t n_kv) {
@@ -715,13 +963,14 @@ size_t prefill_mfma_workspace_bytes(int32_t n_tokens, int32_t n_kv) {
 }
 
 int prefill_mfma_launch(const float * q, int32_t q_stride, const void * k, const void * v, int64_t head_stride,
-                        int32_t n_past, int32_t n_tokens, int32_t n_kv, float scale, float * out, void * workspace,
-                        size_t workspace_bytes, hipStream_t stream) {
+                        int32_t n_past, int32_t n_tokens, int32_t n_kv, float scale, float * out, uint16_t * split,
+                        void * workspace, size_t workspace_bytes, hipStream_t stream) {
     MfmaParams p{};
     p.q = q;
     p.k = static_cast<const _Float16 *>(k);
     p.v = static_cast<const _Float16 *>(v);
     p.out = out;
+    p.split = split;
     p.head_stride = head_stride;
     p.q_stride = q_stride;
     p.n_past = n_past;
@@ -739,6 +988,13 @@ int prefill_mfma_launch(const float * q, int32_t q_stride, const void * k, const
     const size_t stats_bytes = static_cast<size_t>(units) * 2 * kCols * sizeof(PrefillStat);
     if (!workspace || workspace_bytes < kPfFixedBytes + stats_bytes) {
         return fail(QA_ERR_INVALID, "prefill attention: workspace too small (qa_prefill_attn_workspace_bytes)");
+    }
+    // key groups up to 512 workgroups, two per CU (2048 tokens with 8 KV heads): us against the 128-token tiles, 52 tokens
+    // 8.6 / 9.7, 156 11.0 / 17.9, 156 behind 1000 25 / 36, 640 18 / 29, 1037 24 / 36, 1500 35 / 42, 2000 50 / 51, 2500 79 / 60
+    // (every 32 tokens re-read the keys)
+    const int64_t group_wgs = static_cast<int64_t>((n_tokens + kGTok - 1) / kGTok) * n_kv;
+    if (group_wgs <= 512 && !prefill_exact()) {
+        return split ? launch_groups<true>(p, group_wgs, stream) : launch_groups<false>(p, group_wgs, stream);
     }
     const bool can_cut = units <= kPfCutUnits && n_kt_last >= 2 &&
                          workspace_bytes >= prefill_mfma_workspace_bytes(n_tokens, n_kv);
@@ -759,7 +1015,8 @@ int prefill_mfma_launch(const float * q, int32_t q_stride, const void * k, const
     };
     p.queue = reinterpret_cast<uint32_t *>(base);
     if (!prefill_exact()) {
-        hipLaunchKernelGGL(prefill_mfma_kernel<3>, grid_of(resident_grid<3>()), dim3(kPfThreads), 0, stream, p);
+        if (split) hipLaunchKernelGGL((prefill_mfma_kernel<3, true>), grid_of(resident_grid<3>()), dim3(kPfThreads), 0, stream, p);
+        else hipLaunchKernelGGL((prefill_mfma_kernel<3>), grid_of(resident_grid<3>()), dim3(kPfThreads), 0, stream, p);
         QA_LAUNCH_CHECK("prefill_mfma_kernel<3>");
         return QA_OK;
     }

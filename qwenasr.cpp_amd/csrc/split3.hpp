@@ -52,4 +52,18 @@ __device__ inline void store_frag8(uint16_t * out, int k16, int r, int o, const 
     }
 }
 
+// 4 consecutive k (first k % 4 == 0) of row r into the same order
+__device__ inline void store_frag4(uint16_t * out, int k16, int r, int k, float v0, float v1, float v2, float v3) {
+    const float v[4] = {v0, v1, v2, v3};
+    uint16_t part[3][4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) split3_parts(v[e], part[0][e], part[1][e], part[2][e]);
+    uint16_t * d = out + (static_cast<int64_t>(r >> 5) * k16 + (k >> 4)) * 3 * 512 + ((r & 31) + 32 * ((k >> 3) & 1)) * 8 + (k & 7);
+#pragma unroll
+    for (int w = 0; w < 3; ++w) {
+        *reinterpret_cast<uint2 *>(d + w * 512) = make_uint2(part[w][0] | (static_cast<uint32_t>(part[w][1]) << 16),
+                                                             part[w][2] | (static_cast<uint32_t>(part[w][3]) << 16));
+    }
+}
+
 }  // namespace qa
