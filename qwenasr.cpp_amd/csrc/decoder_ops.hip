@@ -130,7 +130,7 @@ struct GemmRowsParams {
     const float * W;          // [N][K]
     const float * X;          // [rows][K]
     float * Y;                // [rows][N]
-    float * partial;          // [ks][rows][N] (ks > 1)
+    float * partial;          // ks > 1: [ks][rows][N], gemm_rows32_kernel [groups][ks][tiles][2][8 rows][2]
     uint32_t * counters;      // [tiles][kGrCounterStride]
     int32_t N, K, rows, ks, slice, accumulate;
     uint32_t x_magic;         // ceil(2^32 / (slice / 4)): X staging index / vectors per token row
@@ -141,6 +141,7 @@ struct GemmRowsParams {
     const double * stats_in;  // [n_stats_in][32]: partial sums of squares of each X row (summed in order)
     double * stats_out;       // [tiles][32]: sums of squares of each stored Y row over the tile's 32 columns
     int32_t n_stats_in, swiglu;
+    int32_t vec4;             // rows of Y hold whole aligned 16-byte groups (gemm_rows32_kernel)
     float eps;
 };
 
@@ -347,8 +348,8 @@ __global__ __launch_bounds__(256) void gemm_rows_kernel(GemmRowsParams p) {
 
 // ---------------------------------------------------------------- skinny GEMM, up to 32 token rows
 // The multi-stream decode step (one token per stream, 32 streams) on v_mfma_f32_32x32x2_f32: a
-// workgroup owns 32 weight rows over one K slice; its 4 waves take the slice's 64-k blocks in turn
-// (wave w: blocks w, w + 4, ...) and are summed through LDS in wave order at the end.
+// workgroup owns 32 weight rows over one K slice; its NW waves take the slice's 64-k blocks in turn
+// (wave w: blocks w, w + NW, ...) and are summed through LDS in wave order at the end.
 // Memory access is what sets the speed here.  The MFMA operand layout puts 32 different rows on the
 // lanes of one load, i.e. 32 B per weight row per instruction, and the memory system moves such
 // loads at ~3 TB/s even with no arithmetic at all; 4 rows x 256 contiguous bytes per instruction
@@ -363,7 +364,13 @@ __global__ __launch_bounds__(256) void gemm_rows_kernel(GemmRowsParams p) {
 // in f32: f32 products and f32 sums, as the f32 path, in another order (5x fewer MFMA cycles: 3 bf16
 // MFMAs per 16 k against 8 f32 ones of 4x the cycles).  hi products go to one accumulator, mid and lo
 // products to the other.
+// What a layer's launches wait for at 32 rows is latency more than bytes (q|k|v of 16.8 MB: 11.7 us, its bytes take
+// 2.6), and of that most was the merge of the K slices through memory: with a lane per token the partial sums and Y
+// went out 16 bytes per 8 KB row.  Partial sums are now stored in thread order (512 contiguous bytes per wave and
+// store) and the threads that finish are mapped to 128 bytes of 8 tokens: bf16 weights, H 2048 / I 6144, q|k|v
+// 14.9 -> 12.3, o 11.1 -> 8.8, down 16.4 -> 14.0 us; f32 weights 18.8 -> 17.0, 14.0 -> 11.1, 20.6 -> 18.1.
 constexpr int kG32Rows = 32;         // weight rows per workgroup (one MFMA block)
+constexpr int kG32Narrow = 24;       // weight rows per tile of the two-tile SwiGLU workgroups
 constexpr int kG32Blk = 64;          // k per block
 constexpr int kG32Ls = kG32Blk + 4;  // LDS row stride (floats)
 constexpr int kG32LsB = kG32Blk + 8; // LDS row stride of bf16 weight rows (elements: 144 B, 16 B aligned)
@@ -401,19 +408,19 @@ __device__ inline void split_bf16x3(const v4f a, const v4f b, u4v & hi, u4v & mi
     }
 }
 
-// T tiles of 32 weight rows per workgroup (T = 2 with bf16 weights and more than 1024 tiles, i.e. the LM
-// head): every X block is loaded, normalised and split into its three bf16 parts once for all T tiles,
-// whose MFMAs then share it.
-template <int P, bool B16, int T>
-__global__ __launch_bounds__(256) void gemm_rows32_kernel(GemmRowsParams p) {
+// NW waves, P blocks in flight per wave, T tiles of R weight rows per workgroup: every X block is loaded, normalised and
+// (B16) split into its three bf16 parts once for all T tiles, whose MFMAs then share it.  R = 24 leaves the last 8
+// rows of each MFMA block unused (SwiGLU only; the rules for all of these are in gemm_rows_plan).
+template <int NW, int P, bool B16, int T, int R>
+__global__ __launch_bounds__(NW * kWave) void gemm_rows32_kernel(GemmRowsParams p) {
 #pragma clang fp contract(off)
-    static_assert(T == 1 || (T == 2 && B16), "two tiles per workgroup with bf16 weights only");
-    // per wave: a block of f32 weight rows, or T blocks of bf16 weight rows; then reused for the cross-wave
-    // sums of T accumulator sets (4 waves x 16 entries x 64 lanes x T)
-    constexpr int kLw = kG32Rows * kG32Ls > T * kG32Rows * kG32LsB / 2 ? kG32Rows * kG32Ls : T * kG32Rows * kG32LsB / 2;
-    static_assert(4 * kLw >= 4 * 16 * kWave * T, "LDS for the cross-wave sums");
-    __shared__ __attribute__((aligned(16))) float lw[4][kLw];
-    __shared__ __attribute__((aligned(16))) float lx[4][kG32Rows * kG32Ls];
+    static_assert(R % 8 == 0 && R <= kG32Rows, "whole load instructions per tile");
+    // per wave: the weight rows and the tokens of a block; then reused for the cross-wave sums of T accumulator sets
+    // (NW waves x 16 entries x 64 lanes x T)
+    constexpr int kLw = B16 ? T * R * kG32LsB / 2 : T * R * kG32Ls, kLx = kG32Rows * kG32Ls;
+    constexpr int kRs = kWave + 1;                                  // row of the cross-wave sums (padded: see total4)
+    static_assert(kLw + kLx >= 16 * kRs * T, "LDS for the cross-wave sums");
+    __shared__ __attribute__((aligned(16))) float lds[NW * (kLw + kLx)];
     __shared__ double s_part[8][32];
     __shared__ float s_scale[32];
     __shared__ int s_last;
@@ -424,14 +431,14 @@ __global__ __launch_bounds__(256) void gemm_rows32_kernel(GemmRowsParams p) {
     const int k_begin = sl * p.slice;
     const int k_len = min(p.slice, p.K - k_begin);                  // multiple of 64
     const int n_blk = k_len / kG32Blk;
-    const int my = (n_blk - wave + 3) / 4;                          // this wave's blocks
+    const int my = (n_blk - wave + NW - 1) / NW;                          // this wave's blocks
     const int last = max(my - 1, 0);
     const bool prenorm = p.norm_w != nullptr;
     // RMSNorm input: thread (token tid % 32, part tid / 32) loads the partial sums of squares k = part,
     // part + 8, ... (at most 16: K <= 4096 with 32-column partials) before any weight load
     double sq[16];
     if (prenorm) {
-        const int tk = threadIdx.x & 31, part = threadIdx.x >> 5;
+        const int tk = threadIdx.x & 31, part = (threadIdx.x >> 5) & 7;
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
             const int k = min(part + 8 * j, p.n_stats_in - 1);
@@ -439,8 +446,9 @@ __global__ __launch_bounds__(256) void gemm_rows32_kernel(GemmRowsParams p) {
         }
     }
     // load lanes: row 4 i + lane / 16 of a block (i = 0..7), k 4 (lane % 16) .. + 3; rows past N re-read
-    // the last row and tokens past `rows` the last token (neither is stored).  SwiGLU tiles hold 16
-    // gate rows and the 16 matching up rows (W = [gate rows; up rows], N = 2 I).
+    // the last row and tokens past `rows` the last token (neither is stored).  SwiGLU tiles hold
+    // R / 2 gate rows and the R / 2 matching up rows (W = [gate rows; up rows], N = 2 I), four gate rows and their
+    // four up rows in turn: both halves of a lane pair (l, l + 32) of the MFMA output.
     const int lr = lane >> 4, lc = 4 * (lane & 15);
     const float * wbase = p.W + k_begin + kG32Blk * wave + lc;
     // bf16 rows: lane loads 8 elements, row 8 i + lane / 8 (i = 0..3) of each tile, k 8 (lane % 8) .. + 7
@@ -449,32 +457,33 @@ __global__ __launch_bounds__(256) void gemm_rows32_kernel(GemmRowsParams p) {
     const float * xbase = p.X + k_begin + kG32Blk * wave + lc;
     const float * nbase = prenorm ? p.norm_w + k_begin + kG32Blk * wave + lc : nullptr;
     auto weight_row = [&](int tile, int line) {
-        const int wr_row = p.swiglu ? (line < 16 ? 16 * tile + line : (p.N >> 1) + 16 * tile + line - 16)
-                                    : tile * kG32Rows + line;
+        const int wr_row = p.swiglu ? (R / 2) * tile + 4 * (line >> 3) + (line & 3) + ((line & 4) ? p.N >> 1 : 0)
+                                    : tile * R + line;
         return static_cast<int64_t>(min(wr_row, p.N - 1)) * p.K;
     };
-    int64_t wrow[8];
+    constexpr int kWt = R / (B16 ? 8 : 4), kWl = T * kWt;           // weight loads per tile, per block
+    int64_t wrow[kWl];
     int xrow[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int line = 4 * i + lr;
-        // B16: entry 4 t + j is row 8 j + lane / 8 of tile T grp + t
-        wrow[i] = B16 ? weight_row(T * grp + (i >> 2), 8 * (i & 3) + lr16) : weight_row(grp, line);
-        xrow[i] = min(line, p.rows - 1) * p.K;
+    for (int i = 0; i < kWl; ++i) {
+        // entry kWt t + j: rows 8 j + lane / 8 (bf16) or 4 j + lane / 16 of tile T grp + t
+        wrow[i] = weight_row(T * grp + i / kWt, B16 ? 8 * (i % kWt) + lr16 : 4 * (i % kWt) + lr);
     }
-    v4f wr[P][8], xr[P][8], nw[P];
-    u4v wb[P][4 * T];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) xrow[i] = min(4 * i + lr, p.rows - 1) * p.K;
+    v4f wr[P][kWl], xr[P][8], nw[P];
+    u4v wb[P][kWl];
     auto load = [&](int u, int b) {
-        const int o = min(b, last) * 4 * kG32Blk;
+        const int o = min(b, last) * NW * kG32Blk;
 #pragma unroll
         for (int i = 0; i < 8; ++i) xr[u][i] = *reinterpret_cast<const v4f *>(xbase + xrow[i] + o);
         if (prenorm) nw[u] = *reinterpret_cast<const v4f *>(nbase + o);
         if constexpr (B16) {
 #pragma unroll
-            for (int i = 0; i < 4 * T; ++i) wb[u][i] = __builtin_nontemporal_load(reinterpret_cast<const u4v *>(wbase16 + wrow[i] + o));
+            for (int i = 0; i < kWl; ++i) wb[u][i] = __builtin_nontemporal_load(reinterpret_cast<const u4v *>(wbase16 + wrow[i] + o));
         } else {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) wr[u][i] = __builtin_nontemporal_load(reinterpret_cast<const v4f *>(wbase + wrow[i] + o));
+            for (int i = 0; i < kWl; ++i) wr[u][i] = __builtin_nontemporal_load(reinterpret_cast<const v4f *>(wbase + wrow[i] + o));
         }
     };
     if (my > 0) {
@@ -487,13 +496,13 @@ __global__ __launch_bounds__(256) void gemm_rows32_kernel(GemmRowsParams p) {
     if (prenorm) {
         // rms_norm_row (text-decoder.cpp:542-557): sum of squares in double, float scale, (x * scale) * w;
         // partial sums are added in a fixed order (k = part + 8 j by j, then the 8 parts in order)
-        const int tk = threadIdx.x & 31, part = threadIdx.x >> 5;
+        const int tk = threadIdx.x & 31, part = (threadIdx.x >> 5) & 7;
         double ss = 0.0;
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
             if (part + 8 * j < p.n_stats_in) ss += sq[j];
         }
-        s_part[part][tk] = ss;
+        if (threadIdx.x < 256) s_part[part][tk] = ss;
         __syncthreads();
         if (threadIdx.x < 32) {
             double tot = 0.0;
@@ -505,9 +514,10 @@ __global__ __launch_bounds__(256) void gemm_rows32_kernel(GemmRowsParams p) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) sc[i] = s_scale[min(4 * i + lr, p.rows - 1)];
     }
-    float * myw = lw[wave];
-    float * myx = lx[wave];
+    float * myw = lds + wave * kLw;
+    float * myx = lds + NW * kLw + wave * kLx;
     const int r = lane & 31, h = lane >> 5;
+    const int ra = min(r, R - 1);   // weight row of the A operand (rows R .. 31 of a tile are not stored)
     v16f acc0[T], acc1[T];
 #pragma unroll
     for (int t = 0; t < T; ++t) { acc0[t] = v16f{}; acc1[t] = v16f{}; }
@@ -520,14 +530,12 @@ __global__ __launch_bounds__(256) void gemm_rows32_kernel(GemmRowsParams p) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) xv[e] = xv[e] * sc[i] * nw[u][e];
             }
-            if constexpr (!B16) *reinterpret_cast<v4f *>(myw + (4 * i + lr) * kG32Ls + lc) = wr[u][i];
             *reinterpret_cast<v4f *>(myx + (4 * i + lr) * kG32Ls + lc) = xv;
         }
-        if constexpr (B16) {
 #pragma unroll
-            for (int i = 0; i < 4 * T; ++i) {
-                *reinterpret_cast<u4v *>(myw16 + ((i >> 2) * kG32Rows + 8 * (i & 3) + lr16) * kG32LsB + lc16) = wb[u][i];
-            }
+        for (int i = 0; i < kWl; ++i) {
+            if constexpr (B16) *reinterpret_cast<u4v *>(myw16 + (8 * i + lr16) * kG32LsB + lc16) = wb[u][i];
+            else *reinterpret_cast<v4f *>(myw + (4 * i + lr) * kG32Ls + lc) = wr[u][i];
         }
         // the block is read back by other lanes of this wave: LDS operations of a wave complete in order
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -542,7 +550,7 @@ __global__ __launch_bounds__(256) void gemm_rows32_kernel(GemmRowsParams p) {
                 split_bf16x3(x0, x1, bh, bm, bl);
 #pragma unroll
                 for (int t = 0; t < T; ++t) {
-                    const u4v a = *reinterpret_cast<const u4v *>(myw16 + (t * kG32Rows + r) * kG32LsB + 16 * s + 8 * h);
+                    const u4v a = *reinterpret_cast<const u4v *>(myw16 + (t * R + ra) * kG32LsB + 16 * s + 8 * h);
                     const bf16x8 av = __builtin_bit_cast(bf16x8, a);
                     acc0[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, __builtin_bit_cast(bf16x8, bh), acc0[t], 0, 0, 0);
                     acc1[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, __builtin_bit_cast(bf16x8, bm), acc1[t], 0, 0, 0);
@@ -556,14 +564,17 @@ __global__ __launch_bounds__(256) void gemm_rows32_kernel(GemmRowsParams p) {
         for (int s = 0; s < 4; ++s) {
             // MFMA step s: k 16 s + 4 h + j (acc0) and 16 s + 8 + 4 h + j (acc1), j = 0..3 -- the same
             // permutation of k for the W (A) and X (B) operands
-            const v4f a0 = *reinterpret_cast<const v4f *>(myw + r * kG32Ls + 16 * s + 4 * h);
-            const v4f a1 = *reinterpret_cast<const v4f *>(myw + r * kG32Ls + 16 * s + 8 + 4 * h);
             const v4f b0 = *reinterpret_cast<const v4f *>(myx + r * kG32Ls + 16 * s + 4 * h);
             const v4f b1 = *reinterpret_cast<const v4f *>(myx + r * kG32Ls + 16 * s + 8 + 4 * h);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                acc0[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[j], b0[j], acc0[0], 0, 0, 0);
-                acc1[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[j], b1[j], acc1[0], 0, 0, 0);
+            for (int t = 0; t < T; ++t) {
+                const v4f a0 = *reinterpret_cast<const v4f *>(myw + (t * R + ra) * kG32Ls + 16 * s + 4 * h);
+                const v4f a1 = *reinterpret_cast<const v4f *>(myw + (t * R + ra) * kG32Ls + 16 * s + 8 + 4 * h);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    acc0[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[j], b0[j], acc0[t], 0, 0, 0);
+                    acc1[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[j], b1[j], acc1[t], 0, 0, 0);
+                }
             }
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -593,90 +604,109 @@ __global__ __launch_bounds__(256) void gemm_rows32_kernel(GemmRowsParams p) {
         if (u < my - full) compute(u);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    // sum the 4 waves (wave order) through LDS: accumulator entry i of lane (r, h) is row
-    // 8 (i / 4) + 4 h + i % 4 of token r (32x32 MFMA output layout); tile t's sums at t 4096
+    // sum the waves (wave order) through LDS: accumulator entry i of lane (r, h) is row 8 (i / 4) + 4 h + i % 4 of
+    // token r (32x32 MFMA output layout)
     __syncthreads();
-    float * red = &lw[0][0];
+    float * red = lds;
 #pragma unroll
     for (int t = 0; t < T; ++t) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) red[((t * 4 + wave) * 16 + i) * kWave + lane] = acc0[t][i] + acc1[t][i];
+        for (int i = 0; i < 16; ++i) red[((t * NW + wave) * 16 + i) * kRs + lane] = acc0[t][i] + acc1[t][i];
     }
     __syncthreads();
-    auto entry = [&](int t, int i) {
-        float a = red[(t * 64 + i) * kWave + lane];
+    const int tid = static_cast<int>(threadIdx.x);
+    // rows 4 c .. 4 c + 3 of tile t for one token
+    auto total4 = [&](int t, int c, int token) {
+        v4f a;
+        const float * q = red + (t * NW * 16 + 4 * (c >> 1)) * kRs + 32 * (c & 1) + token;
 #pragma unroll
-        for (int v = 1; v < 4; ++v) a += red[((t * 4 + v) * 16 + i) * kWave + lane];
+        for (int j = 0; j < 4; ++j) {
+            a[j] = q[j * kRs];
+#pragma unroll
+            for (int v = 1; v < NW; ++v) a[j] += q[(v * 16 + j) * kRs];
+        }
         return a;
     };
-    const int tk = r;   // token of this lane's outputs
     if (p.swiglu) {
-        // one slice (ks = 1): waves 0 and 1 own gate rows 8 w + 4 h + 0..3 (entries 4 w + j) and their up
-        // rows 16 + 8 w + 4 h + 0..3 (entries 4 w + 8 + j) of each tile; silu(gate) * up as
+        // one slice (ks = 1): consecutive threads take the 4-row groups of one token; silu(gate) * up as
         // text-decoder.cpp:602
-        if (wave < 2 && tk < p.rows) {
-            const int I = p.N >> 1;
+        constexpr int G = R / 8;                                     // groups of 4 gate rows per tile
+        const int tk = tid / (T * G), t = tid % (T * G) / G, a = tid % G;
+        if (tk < p.rows) {
+            const int I = p.N >> 1, c = (R / 2) * (T * grp + t) + 4 * a;
+            float * y = p.Y + static_cast<int64_t>(tk) * I + c;
+            const v4f gate = total4(t, 2 * a, tk), up = total4(t, 2 * a + 1, tk);
+            v4f o;
 #pragma unroll
-            for (int t = 0; t < T; ++t) {
-                const int c = 16 * (T * grp + t) + 8 * wave + 4 * h;
-                float * y = p.Y + static_cast<int64_t>(tk) * I + c;
+            for (int j = 0; j < 4; ++j) o[j] = (gate[j] / (1.0f + expf(-gate[j]))) * up[j];
+            if (p.vec4) {
+                if (c < I) *reinterpret_cast<v4f *>(y) = o;
+            } else {
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    const float g = entry(t, 4 * wave + j), u = entry(t, 4 * wave + 8 + j);
-                    if (c + j < I) y[j] = (g / (1.0f + expf(-g))) * u;
+                    if (c + j < I) y[j] = o[j];
                 }
             }
         }
         return;
     }
-    // wave w owns entries 4 w .. 4 w + 3 of each tile: rows 8 w + 4 h + 0..3 of token r
+    // the first 256 threads: thread tid finishes rows 4 (tid % 8) + 0..3 of each tile for token tid / 8, so that a
+    // wave stores 128 contiguous bytes of 8 tokens
+    const int tk = tid >> 3, cg = tid & 7;
+    const bool mine = NW == 4 || tid < 256;
     v4f sv[T];
     int nr[T];
     bool live[T];
 #pragma unroll
     for (int t = 0; t < T; ++t) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) sv[t][j] = entry(t, 4 * wave + j);
-        nr[t] = (T * grp + t) * kG32Rows + 8 * wave + 4 * h;
-        live[t] = tk < p.rows && nr[t] < p.N;
+        sv[t] = total4(t, cg, tk & 31);
+        nr[t] = (T * grp + t) * kG32Rows + 4 * cg;
+        live[t] = mine && tk < p.rows && nr[t] < p.N;
     }
-    // store (or accumulate) the final values of tile t; with stats_out also the tile's per-token sum of
-    // squares of the stored values (a workgroup-uniform step: every thread of the workgroup calls it)
-    // the old values of tile t's 4 outputs of this lane (accumulate), read by 4 loads issued together
-    // (addresses clamped to the matrix, no branch), so that they cost one round trip
+    // the old values of tile t's 4 outputs of this thread (accumulate), loaded together (addresses clamped to the
+    // matrix, no branch per lane), so that they cost one round trip
     auto old_values = [&](int t) {
         v4f o = v4f{};
         if (p.accumulate) {
             const float * y = p.Y + static_cast<int64_t>(min(tk, p.rows - 1)) * p.N;
+            if (p.vec4) {
+                o = *reinterpret_cast<const v4f *>(y + min(nr[t], p.N - 4));
+            } else {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) o[i] = y[min(nr[t] + i, p.N - 1)];
+                for (int i = 0; i < 4; ++i) o[i] = y[min(nr[t] + i, p.N - 1)];
+            }
         }
         return o;
     };
+    // store (or accumulate) the final values of tile t; with stats_out also the tile's per-token sum of
+    // squares of the stored values (a workgroup-uniform step: every thread of the workgroup calls it)
     auto finish = [&](int t, v4f v, v4f old) {
         double ss = 0.0;
         if (live[t]) {
             float * y = p.Y + static_cast<int64_t>(tk) * p.N + nr[t];
+            if (p.accumulate) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = old[i] + v[i];
+            }
+            if (p.vec4) *reinterpret_cast<v4f *>(y) = v;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 if (nr[t] + i < p.N) {
-                    const float o = p.accumulate ? old[i] + v[i] : v[i];
-                    y[i] = o;
-                    ss += static_cast<double>(o) * o;
+                    if (!p.vec4) y[i] = v[i];
+                    ss += static_cast<double>(v[i]) * v[i];
                 }
             }
         }
         if (p.stats_out) {
-            double * sst = &s_part[0][0];                           // [4 waves][2 halves][32 tokens]
-            sst[(2 * wave + h) * 32 + tk] = ss;
+            if (mine) s_part[cg][tk] = ss;
             __syncthreads();
             if (threadIdx.x < 32) {
                 double tot = 0.0;
 #pragma unroll
-                for (int q = 0; q < 8; ++q) tot += sst[q * 32 + threadIdx.x];
+                for (int q = 0; q < 8; ++q) tot += s_part[q][threadIdx.x];
                 p.stats_out[32 * (T * grp + t) + threadIdx.x] = tot;
             }
-            __syncthreads();   // sst is written again by the next tile's step
+            __syncthreads();   // s_part is written again by the next tile's step
         }
     };
     if (p.ks == 1) {
@@ -687,17 +717,20 @@ __global__ __launch_bounds__(256) void gemm_rows32_kernel(GemmRowsParams p) {
         for (int t = 0; t < T; ++t) finish(t, sv[t], old[t]);
         return;
     }
-    // publish (partial rows padded to whole 4-row groups), then the last slice of the tile group merges in
-    // slice order -- the same protocol as gemm_rows_kernel
-    const int np = (p.N + 3) / 4 * 4;
+    // publish, each store of a wave one contiguous block, then the last slice of the tile group merges in slice order
+    // -- the same protocol as gemm_rows_kernel
+    const int n_pub = 8 * p.rows;                                    // threads with a live token
+    auto slot = [&](int slice, int t, int q) {
+        const int64_t block = ((static_cast<int64_t>(grp) * p.ks + slice) * T + t) * 2 + q;
+        return reinterpret_cast<uint64_t *>(p.partial) + block * n_pub + min(tid, n_pub - 1);
+    };
 #pragma unroll
     for (int t = 0; t < T; ++t) {
-        if (live[t]) {
-            uint64_t * q = reinterpret_cast<uint64_t *>(p.partial + (static_cast<int64_t>(sl) * p.rows + tk) * np + nr[t]);
+        if (tid < n_pub) {
             const uint64_t lo = static_cast<uint64_t>(__float_as_uint(sv[t][0])) | (static_cast<uint64_t>(__float_as_uint(sv[t][1])) << 32);
             const uint64_t hi = static_cast<uint64_t>(__float_as_uint(sv[t][2])) | (static_cast<uint64_t>(__float_as_uint(sv[t][3])) << 32);
-            __hip_atomic_store(q, lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(q + 1, hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(slot(sl, t, 0), lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(slot(sl, t, 1), hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -710,19 +743,16 @@ __global__ __launch_bounds__(256) void gemm_rows32_kernel(GemmRowsParams p) {
     }
     __syncthreads();
     if (!s_last) return;
-    const int tt = min(tk, p.rows - 1);
 #pragma unroll
     for (int t = 0; t < T; ++t) {
-        const int nn = min(nr[t], np - 4);
         // one round of loads: the plan merges at most kG32MaxSlices slices; no loop, whose back edge would
         // make the compiler wait for earlier loads before reusing their registers
         uint64_t v[kG32MaxSlices][2];
 #pragma unroll
         for (int u = 0; u < kG32MaxSlices; ++u) {
             const int k = min(u, p.ks - 1);
-            const uint64_t * q = reinterpret_cast<const uint64_t *>(p.partial + (static_cast<int64_t>(k) * p.rows + tt) * np + nn);
-            v[u][0] = __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            v[u][1] = __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            v[u][0] = __hip_atomic_load(slot(k, t, 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            v[u][1] = __hip_atomic_load(slot(k, t, 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         const v4f old = old_values(t);   // issued behind the partials' loads, waited for with them
         float sum[4] = {0.f, 0.f, 0.f, 0.f};
@@ -742,7 +772,9 @@ struct GemmRowsPlan {
     int ks, slice, tiles;
     bool rows32;     // gemm_rows32_kernel (else gemm_rows_kernel)
     int depth;       // blocks in flight per wave (gemm_rows32_kernel)
-    int tpw;         // tiles per workgroup (gemm_rows32_kernel: 2 with bf16 weights, an even tile count and > 1024 tiles)
+    int waves;       // per workgroup (gemm_rows32_kernel)
+    int tpw;         // tiles per workgroup (gemm_rows32_kernel)
+    int tile_rows;   // weight rows per tile (gemm_rows32_kernel: 32, or 24 for two-tile SwiGLU workgroups)
 };
 
 // tuning overrides of the <= 32-row plan: QA_GR32_WGS (workgroup target, default 256) and QA_GR32_DEPTH
@@ -758,13 +790,32 @@ GemmRowsPlan gemm_rows_plan(int32_t N, int32_t K, int32_t rows, bool one_slice =
     static const int forced_depth = env_int("QA_GR32_DEPTH", 0);
     static const int forced_tpw = env_int("QA_GR32_TPW", 0);
     if (rows <= kG32Rows && K % kG32Blk == 0) {
-        // ~256 workgroups at least (one per CU); a K slice keeps >= 4 blocks (one per wave) and at most
-        // 8 slices are merged.  Two blocks in flight per wave when the grid is one workgroup per CU (the
-        // register file then holds 2 waves per SIMD either way), one when there are more workgroups.
+        // ~256 workgroups at least (one per CU); a K slice keeps >= 4 blocks (one per 4 waves) and at most
+        // 8 slices are merged.  f32 weights: two blocks in flight per wave when the grid is one workgroup per CU
+        // (the register file then holds 2 waves per SIMD either way), one when there are more workgroups.
+        // bf16 weights: one block in flight, and 8 waves instead of 4 when the grid is one workgroup per CU (32 rows:
+        // q|k|v 12.3 -> 11.7 us, o 8.8 -> 8.2, down 14.0 -> 12.9, H 1024 gate|up 10.2 -> 8.9; f32 weights time the
+        // same either way, 16.3-17.0, 11.1, 18.1, and keep the order of their sums).
         // With bf16 weights and more than 1024 tiles (the LM head) a workgroup takes two tiles, which
         // share each X block and its split (config-4 step: LM head 0.198 -> 0.171 ms); with fewer tiles
         // the grid would drop below two workgroups per CU (layer projections 1.95 -> 2.40 ms per step).
+        // A SwiGLU launch is not cut along K, so 257 to 512 tiles would put two workgroups, which read all of X each, on
+        // some CUs and one on the others.  With bf16 weights two tiles of 24 rows per workgroup give every CU one
+        // workgroup that reads X once (N = 12288: 256 workgroups, 23.0 -> 18.3 us; on f32 weights, where the matrix
+        // cores carry the wasted rows too, 32.6 and 32.0: left as it was).  Past 12288 rows the second workgroup per
+        // CU is back and the 32-row tiles waste no MFMA rows.
         pl.rows32 = true;
+        pl.tile_rows = kG32Rows;
+        if (b16 && one_slice && N > 256 * kG32Rows && N <= 256 * 2 * kG32Narrow) {
+            pl.tile_rows = kG32Narrow;
+            pl.tpw = 2;
+            pl.tiles = 2 * ((N + 2 * kG32Narrow - 1) / (2 * kG32Narrow));
+            pl.ks = 1;
+            pl.slice = K;
+            pl.depth = 1;
+            pl.waves = 8;
+            return pl;
+        }
         pl.tiles = (N + kG32Rows - 1) / kG32Rows;
         pl.tpw = b16 && pl.tiles % 2 == 0 && (pl.tiles > 1024 || forced_tpw == 2) && forced_tpw != 1 ? 2 : 1;
         const int groups = pl.tiles / pl.tpw;
@@ -772,7 +823,8 @@ GemmRowsPlan gemm_rows_plan(int32_t N, int32_t K, int32_t rows, bool one_slice =
         if (groups > kGrMaxTiles || one_slice) ks = 1;             // counters exist for kGrMaxTiles groups
         pl.slice = ((K + ks - 1) / ks + kG32Blk - 1) / kG32Blk * kG32Blk;
         pl.ks = (K + pl.slice - 1) / pl.slice;
-        pl.depth = forced_depth == 1 || forced_depth == 2 ? forced_depth : groups * pl.ks <= 256 ? 2 : 1;
+        pl.waves = b16 && pl.tpw == 1 && groups * pl.ks <= 256 ? 8 : 4;
+        pl.depth = b16 && pl.tpw == 1 ? 1 : forced_depth == 1 || forced_depth == 2 ? forced_depth : groups * pl.ks <= 256 ? 2 : 1;
         return pl;
     }
     pl.tiles = (N + kGrTile - 1) / kGrTile;
@@ -1010,9 +1062,12 @@ int pack_bf16_launch(const float * src, int64_t n, uint16_t * dst, uint32_t * in
 
 size_t gemm_rows_workspace_bytes(int32_t N, int32_t K, int32_t rows) {
     if (N <= 0 || N > kGrMaxTiles * kGrTile || K <= 0 || rows <= 0 || rows > kGrMaxRows || K % 32 != 0) return 0;
-    // the larger of the f32-weight and bf16-weight plans (their slice counts differ)
+    // the larger of the f32-weight and bf16-weight plans (their slice counts differ), for whole tiles of 32 rows; more
+    // than 32 rows also cover every smaller row count
     const int ks = std::max(gemm_rows_plan(N, K, rows).ks, gemm_rows_plan(N, K, rows, false, true).ks);
-    const size_t partial = ks > 1 ? static_cast<size_t>(ks) * rows * ((N + 3) / 4 * 4) * sizeof(float) : 0;
+    const int64_t np = rows <= kG32Rows ? (N + kG32Rows - 1) / kG32Rows * kG32Rows : (N + 3) / 4 * 4;
+    const size_t partial = ks > 1 ? static_cast<size_t>(ks) * rows * np * sizeof(float) : 0;
+    if (rows > kG32Rows) return std::max(kGrCounterBytes + partial, gemm_rows_workspace_bytes(N, K, kG32Rows));
     return kGrCounterBytes + partial;
 }
 
@@ -1066,17 +1121,21 @@ int gemm_rows_launch(const float * W, int32_t N, int32_t K, const float * X, int
         p.swiglu = fusion->swiglu ? 1 : 0;
     }
     if (pl.rows32) {
+        p.vec4 = (p.swiglu ? N / 2 : N) % 4 == 0 && reinterpret_cast<uintptr_t>(Y) % 16 == 0;
         const dim3 grid(static_cast<unsigned>(pl.tiles / pl.tpw * pl.ks));
         p.W16 = W16;
-        if (W16 && pl.tpw == 2) {
-            if (pl.depth == 2) hipLaunchKernelGGL((gemm_rows32_kernel<2, true, 2>), grid, dim3(256), 0, stream, p);
-            else hipLaunchKernelGGL((gemm_rows32_kernel<1, true, 2>), grid, dim3(256), 0, stream, p);
+        const dim3 block(static_cast<unsigned>(pl.waves * kWave));
+        if (pl.tile_rows == kG32Narrow) {
+            hipLaunchKernelGGL((gemm_rows32_kernel<8, 1, true, 2, kG32Narrow>), grid, block, 0, stream, p);
+        } else if (W16 && pl.tpw == 2) {
+            if (pl.depth == 2) hipLaunchKernelGGL((gemm_rows32_kernel<4, 2, true, 2, kG32Rows>), grid, block, 0, stream, p);
+            else hipLaunchKernelGGL((gemm_rows32_kernel<4, 1, true, 2, kG32Rows>), grid, block, 0, stream, p);
         } else if (W16) {
-            if (pl.depth == 2) hipLaunchKernelGGL((gemm_rows32_kernel<2, true, 1>), grid, dim3(256), 0, stream, p);
-            else hipLaunchKernelGGL((gemm_rows32_kernel<1, true, 1>), grid, dim3(256), 0, stream, p);
+            if (pl.waves == 8) hipLaunchKernelGGL((gemm_rows32_kernel<8, 1, true, 1, kG32Rows>), grid, block, 0, stream, p);
+            else hipLaunchKernelGGL((gemm_rows32_kernel<4, 1, true, 1, kG32Rows>), grid, block, 0, stream, p);
         } else {
-            if (pl.depth == 2) hipLaunchKernelGGL((gemm_rows32_kernel<2, false, 1>), grid, dim3(256), 0, stream, p);
-            else hipLaunchKernelGGL((gemm_rows32_kernel<1, false, 1>), grid, dim3(256), 0, stream, p);
+            if (pl.depth == 2) hipLaunchKernelGGL((gemm_rows32_kernel<4, 2, false, 1, kG32Rows>), grid, block, 0, stream, p);
+            else hipLaunchKernelGGL((gemm_rows32_kernel<4, 1, false, 1, kG32Rows>), grid, block, 0, stream, p);
         }
         QA_LAUNCH_CHECK("gemm_rows32_kernel");
         return QA_OK;
