@@ -468,7 +468,7 @@ def prefill_attn_roofline(cfg, T: int, fam_ms: dict):
 
 
 def prefill_gemm_roofline(cfg, T: int, fam_ms: dict):
-    """The bf16-exact prefill projections (gemm_split3: bf16 MFMA over the three-part split of each input, so
+    """The bf16-exact prefill projections (gemm_prefill: bf16 MFMA over the three-part split of each input, so
     3 x 2 T params FLOPs of MFMA work per layer) from the projection family's time, which also holds the
     RMSNorm and split passes: a lower bound on the GEMM's own rate."""
     H, QD, KD, I = cfg.hidden, cfg.n_heads * cfg.head_dim, cfg.n_kv_heads * cfg.head_dim, cfg.intermediate
@@ -478,7 +478,7 @@ def prefill_gemm_roofline(cfg, T: int, fam_ms: dict):
     tf = flop / (ms * 1e-3) / 1e12
     return {"bound": "mfma", "achieved": round(tf, 1), "peak": MFMA_F16_PEAK_TFLOPS, "unit": "TFLOP/s",
             "frac": round(tf / MFMA_F16_PEAK_TFLOPS, 4), "traffic": None,
-            "kernel": "gemm_split3_kernel (bf16 MFMA over the split input, SwiGLU fused), the prefill's projection "
+            "kernel": "gemm_prefill_kernel (bf16 MFMA over the split input, SwiGLU fused), the prefill's projection "
                       "family (with its RMSNorm and split passes)", "flop_per_layer": round(flop / cfg.n_layers),
             "positions": T, "ms": ms}
 

@@ -276,7 +276,7 @@ bool skinny_path(const qa_decoder * d, int32_t rows, int32_t in_dim) {
 int sgemm(qa_decoder * d, const float * W, int32_t out_dim, int32_t in_dim, const float * X, int32_t rows, float * Y,
           float beta) {
     // Y[rows][out] (+)= X[rows][in] * W[out][in]^T on f32 weights.  Up to kSkinnyRows rows (multi-stream decode,
-    // short prefills) the weights are streamed once by the skinny MFMA GEMM; longer prefills run rocBLAS sgemm.
+    // prompts the prompt GEMM does not take) the weights are streamed once by the skinny MFMA GEMM; longer ones run rocBLAS.
     if (skinny_path(d, rows, in_dim)) {
         return gemm_rows_launch(W, out_dim, in_dim, X, rows, Y, beta != 0.0f, d->gr_ws, d->gr_ws_bytes, d->stream);
     }

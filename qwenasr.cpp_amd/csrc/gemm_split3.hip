@@ -1,4 +1,5 @@
-// Prefill projections on bf16-exact weights, gfx950 (bf16 MFMA, v_mfma_f32_32x32x16_bf16).
+// qa_gemm_split3_bf16: Y = X W^T on bf16-exact weights over a split input, gfx950 (bf16 MFMA, v_mfma_f32_32x32x16_bf16).
+// (The decoder's own prompts run gemm_prefill.hip.)
 //
 // Replaces linear_ggml with PREC_F32 (text-decoder.cpp:83-90) for T > 32 rows when the f32 weights are
 // bf16-exact (their low 16 bits are zero, as in every checkpoint converted from the released bf16 weights,
