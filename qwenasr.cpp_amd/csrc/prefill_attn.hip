@@ -387,9 +387,11 @@ __device__ inline void f32mfma_block(const RowsParams & p, float * lds, int kvh,
             for (int o = 1; o < KG; ++o) {
                 const int w = (o - 1) * kWaves + gw;
                 const float mo = sm[w * kWave + lane];
-                if (mo == -INFINITY) continue;                       // no key of the group before this query
                 const float m_new = fmaxf(m_run, mo);
-                const float ca = expf(m_run - m_new), cb = expf(mo - m_new);
+                // a maximum of -inf weighs 0 and is still added: fmaxf passes over a NaN, so a group whose only scores
+                // for this query are NaN has that maximum too, and 0 * NaN keeps the NaN
+                const float ca = m_run == -INFINITY ? 0.0f : expf(m_run - m_new);
+                const float cb = mo == -INFINITY ? 0.0f : expf(mo - m_new);
                 l_run = l_run * static_cast<double>(ca) + sl[w * kWave + lane] * static_cast<double>(cb);
                 m_run = m_new;
 #pragma unroll

@@ -35,3 +35,36 @@ def test_f32_prefill_equals_row_kernel(qa, n_past, T):
     d = outs[0] - outs[1]
     assert np.isfinite(d).all()
     assert np.abs(d).max() <= 2e-5 and np.linalg.norm(d) <= 2e-6 * np.linalg.norm(outs[1]), (np.abs(d).max(),)
+
+
+@pytest.mark.parametrize("entry,T,bad", [("causal", 33, 32), ("causal", 97, 64), ("causal", 130, 96), ("cache", 33, 32),
+                                         ("cache", 64, 5), ("cache", 1300, 32)])
+def test_f32_prefill_keeps_nan(qa, entry, T, bad):
+    """A NaN in key row `bad` of KV head 3 reaches every query that attends it, also the one that sees no other key of
+    its key group (the query at the key's own position, where the key opens a tile); nothing else moves by a bit."""
+    assert qa.device_count() > 0, "no HIP device: GPU tests need the MI355X"
+    rng = np.random.default_rng(T + bad)
+    q = qa.DeviceArray.from_numpy(rng.standard_normal((T, 2048)).astype(np.float32))
+    k, v = (rng.standard_normal((8, T, 128)).astype(np.float32) for _ in range(2))
+    outs = []
+    for poisoned in (False, True):
+        if poisoned:
+            k[3, bad, 17] = np.nan
+        out = qa.DeviceArray((T, 2048))
+        print(f"f32 prefill entry={entry} T={T} NaN key {bad if poisoned else None}", flush=True)
+        if entry == "causal":
+            dk, dv = (qa.DeviceArray.from_numpy(np.ascontiguousarray(a.transpose(1, 0, 2))) for a in (k, v))
+            qa.check(qa.lib.qa_causal_attn_f32(q.ptr, dk.ptr, dv.ptr, T, 16, 8, 128 ** -0.5, out.ptr, None))
+        else:
+            lay = qa.KvLayout(1, 1, 8, 128, T, qa.QA_CACHE_F32)
+            cache = qa.DeviceArray.from_numpy(np.stack([k, v]))
+            qa.check(qa.lib.qa_prefill_attn(q.ptr, cache.ptr, C.byref(lay), 0, 0, 0, T, 16, 128 ** -0.5, out.ptr, None, 0,
+                                            None))
+        qa.synchronize()
+        outs.append(out.numpy().reshape(T, 16, 128))
+    clean, got = outs
+    assert np.isfinite(clean).all()
+    hit = np.zeros(clean.shape, bool)
+    hit[bad:, 6:8] = True
+    assert np.isnan(got[hit]).all(), np.argwhere(~np.isnan(got[bad:, 6:8]).all(axis=(1, 2)))[:4].ravel() + bad
+    np.testing.assert_array_equal(got[~hit].view(np.uint32), clean[~hit].view(np.uint32))
