@@ -655,8 +655,9 @@ __device__ inline void run_item(const MfmaParams & p, const Item & it, _Float16 
 // tiles (32 keys) in turn, group kg the tiles kg, kg + 4, ..., each staged in LDS by its two waves, with the online
 // softmax of the single pass; at the end the four states of a head are merged through LDS, in group order, every wave
 // taking a quarter of the dims.  No queue, no cut tiles, no workspace.
-// What it is for: up to about 2000 tokens the 128-token tiles above are few (16 at 156 tokens) and each walks its key
-// tiles in sequence, 3.4 us a tile of 64 keys, with a merge of cut tiles across workgroups behind it.
+// What it is for: up to about 1000 tokens (2000 with few cached positions) the 128-token tiles above are few (16 at 156
+// tokens) and each walks its key tiles in sequence, 3.4 us a tile of 64 keys, with a merge of cut tiles across workgroups
+// behind it.
 constexpr int kGTok = 32;                        // query tokens per workgroup
 constexpr int kGKeys = 32;                       // keys per tile
 constexpr int kGVS = 48;                         // V^T row stride (halfs): 24 dwords, conflict-free like kVS
@@ -989,11 +990,17 @@ int prefill_mfma_launch(const float * q, int32_t q_stride, const void * k, const
     if (!workspace || workspace_bytes < kPfFixedBytes + stats_bytes) {
         return fail(QA_ERR_INVALID, "prefill attention: workspace too small (qa_prefill_attn_workspace_bytes)");
     }
-    // key groups up to 512 workgroups, two per CU (2048 tokens with 8 KV heads): us against the 128-token tiles, 52 tokens
-    // 8.6 / 9.7, 156 11.0 / 17.9, 156 behind 1000 25 / 36, 640 18 / 29, 1037 24 / 36, 1500 35 / 42, 2000 50 / 51, 2500 79 / 60
-    // (every 32 tokens re-read the keys)
+    // Key groups: a CU holds one of their workgroups (LDS), and every 32 tokens re-read all keys before them, so the rule
+    // looks at both counts.  us against the 128-token tiles (8 KV heads):
+    //   up to 256 workgroups, one round (1024 tokens): 156 tokens 11.2 / 17.8, 1024 23.0 / 33.6, 156 behind 1000
+    //   24.7 / 36.0, 1024 behind 8000 130 / 135; far behind, the tiles' walk is as short: 16 behind 16000 230 / 216, 512
+    //   behind 30000 414 / 404;
+    //   a second round (up to 2048 tokens) pays while it is short: 2048 45 / 48, 2048 behind 100 48.5 / 49.9, 1500 behind
+    //   500 44.8 / 47.3; then the keys are read too often: 2048 behind 250 52.2 / 51.5, 1280 behind 1000 51.2 / 51.2, 1280
+    //   behind 4000 127 / 90, 2048 behind 16000 460 / 253; a third never does: 2500 71 / 55.
     const int64_t group_wgs = static_cast<int64_t>((n_tokens + kGTok - 1) / kGTok) * n_kv;
-    if (group_wgs <= 512 && !prefill_exact()) {
+    const int group_keys = group_wgs <= 256 ? 12288 : group_wgs <= 512 ? 2176 : 0;    // past and new positions
+    if (n_past + n_tokens <= group_keys && !prefill_exact()) {
         return split ? launch_groups<true>(p, group_wgs, stream) : launch_groups<false>(p, group_wgs, stream);
     }
     const bool can_cut = units <= kPfCutUnits && n_kt_last >= 2 &&
