@@ -384,7 +384,7 @@ __device__ inline void f32mfma_block(const RowsParams & p, float * lds, int kvh,
         }
         __syncthreads();
         if (kg == 0) {
-            for (int o = 1; o < KG; ++o) {
+            for (int o = 1; o < min(KG, n_tiles); ++o) {             // (groups from n_tiles on had no tile)
                 const int w = (o - 1) * kWaves + gw;
                 const float mo = sm[w * kWave + lane];
                 const float m_new = fmaxf(m_run, mo);
@@ -446,9 +446,13 @@ int launch_f32_groups(const RowsParams & p, int n_kv_heads, hipStream_t stream) 
 // workgroups pay for their start, the merge and the K/V tiles that more blocks re-read, so the groups go down as the
 // grid grows past about 2.5 and 3.4 workgroups per CU.  us by groups 4 / 2 / 1: 156 tokens 16 / 19 / 27 (42 before), 156
 // behind 1000 63 / 102 / 180 (366), 640 37 / 58 / 101 (121), 1037 79 / 94 / 164 (193), 1500 140 / 133 / 230 (269), 2500
-// 344 / 315 / 385 (441), 3000 455 / 431 / 464 (520), 3913 774 / 661 / 642 (690).
+// 344 / 315 / 385 (441), 3000 455 / 431 / 464 (520), 3913 774 / 661 / 642 (690).  Behind 1000 cached positions the lines
+// lie a little lower (1100 tokens 219 / 202 / 321, 2500 563 / 550 / 534), behind 4000 about the same (1280 669 / 706 / 794,
+// 3456 1910 / 1781 / 1669); the kernel before them took 549, 758, 1499 and 1855 there.
+// With one key tile there is nothing to share out: 16 tokens 8.3 on four groups, 6.8 on two (7.6).
 int launch_f32mfma(const RowsParams & p, int n_kv_heads, hipStream_t stream) {
     auto workgroups = [&](int queries) { return (p.n_tokens + queries - 1) / queries * n_kv_heads; };
+    if (p.n_past + p.n_tokens <= kF32Tile) return launch_f32_groups<2, 2>(p, n_kv_heads, stream);
     if (workgroups(16) <= 640) return launch_f32_groups<4, 1>(p, n_kv_heads, stream);
     if (workgroups(32) <= 864) return launch_f32_groups<2, 2>(p, n_kv_heads, stream);
     return launch_f32_groups<1, 2>(p, n_kv_heads, stream);

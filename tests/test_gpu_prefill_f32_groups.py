@@ -2,6 +2,7 @@
 four, two and one groups of waves, and the prompt lengths where the number of groups changes."""
 import ctypes as C
 import os
+import time
 
 import numpy as np
 import pytest
@@ -68,3 +69,24 @@ def test_f32_prefill_keeps_nan(qa, entry, T, bad):
     hit[bad:, 6:8] = True
     assert np.isnan(got[hit]).all(), np.argwhere(~np.isnan(got[bad:, 6:8]).all(axis=(1, 2)))[:4].ravel() + bad
     np.testing.assert_array_equal(got[~hit].view(np.uint32), clean[~hit].view(np.uint32))
+
+
+def test_f32_prefill_of_one_key_tile_is_short(qa):
+    """16 positions are one key tile, which no key group shares: 6.8 us against 8.1 us for 33 positions (on four groups
+    both took 8.3)."""
+    us = []
+    for T in (16, 33):
+        lay = qa.KvLayout(1, 1, 8, 128, T, qa.QA_CACHE_F32)
+        cache, q, out = qa.DeviceArray((2, 8, T, 128)), qa.DeviceArray((T, 2048)), qa.DeviceArray((T, 2048))
+        args = (q.ptr, cache.ptr, C.byref(lay), 0, 0, 0, T, 16, 128 ** -0.5, out.ptr, None, 0, None)
+        got = []
+        for _ in range(21):
+            qa.synchronize()
+            t = time.perf_counter()
+            for _ in range(200):
+                qa.check(qa.lib.qa_prefill_attn(*args))
+            qa.synchronize()
+            got.append((time.perf_counter() - t) / 200 * 1e6)
+        us.append(sorted(got)[5])
+    print(f"f32 prefill: 16 positions {us[0]:.2f} us, 33 positions {us[1]:.2f} us", flush=True)
+    assert us[0] < 0.93 * us[1]
