@@ -72,6 +72,7 @@ struct qa_decoder {
     float * out_p = nullptr;            // the LM head packed like DevLayer::qkv_p
     std::vector<void *> weight_allocs;
     std::vector<void *> b16_allocs;     // the bf16 weight copies (freed again if the model is not exact)
+    std::vector<void *> prompt_allocs;  // DevLayer::qkv3 .. down3, given back when something else needs the memory
     void * cache = nullptr;
     qa_kv_layout layout{};
     int32_t * d_lens = nullptr;
@@ -183,6 +184,7 @@ void free_acts(qa_decoder * d) {
     d->pf_ws = nullptr;
     d->pf_ws_bytes = 0;
     d->xstats = nullptr;
+    d->gu = nullptr;
     d->xf = nullptr;
     d->actf = nullptr;
     d->partial = nullptr;
@@ -213,8 +215,20 @@ bool prompt_ready(const qa_decoder * d) {
     return !d->layers.empty() && (d->layers[0].qkv16 || d->layers[0].qkv3) && prompt_shapes(d);
 }
 
-int ensure_rows(qa_decoder * d, int32_t rows) {
-    if (rows <= d->cap_rows) return QA_OK;
+// Gives the prompt copies of f32 weights back after an allocation failed; the activations are laid out again by the
+// next ensure_rows (prompts then run on sgemm, which needs other buffers).
+bool drop_prompt_copies(qa_decoder * d) {
+    (void)hipGetLastError();
+    if (d->prompt_allocs.empty()) return false;
+    (void)hipStreamSynchronize(d->stream);
+    for (void * p : d->prompt_allocs) (void)hipFree(p);
+    d->prompt_allocs.clear();
+    for (DevLayer & L : d->layers) L.qkv3 = L.o3 = L.gu3 = L.down3 = nullptr;
+    free_acts(d);
+    return true;
+}
+
+int alloc_rows(qa_decoder * d, int32_t rows) {
     (void)hipStreamSynchronize(d->stream);
     free_acts(d);
     const size_t H = d->cfg.hidden, QD = static_cast<size_t>(d->cfg.n_heads) * kHeadDim,
@@ -267,6 +281,12 @@ int ensure_rows(qa_decoder * d, int32_t rows) {
     }
     d->cap_rows = rows;
     return QA_OK;
+}
+
+int ensure_rows(qa_decoder * d, int32_t rows) {
+    if (rows <= d->cap_rows) return QA_OK;
+    const int rc = alloc_rows(d, rows);
+    return rc == QA_ERR_ALLOC && drop_prompt_copies(d) ? alloc_rows(d, rows) : rc;
 }
 
 bool skinny_path(const qa_decoder * d, int32_t rows, int32_t in_dim) {
@@ -662,16 +682,28 @@ int pack_weights_bf16(qa_decoder * d) {
 // f32 weights: the three-part split of every projection in fragment order, 6 bytes per weight (8.5 GB for the 1.7B
 // model), with which a prompt's projections run on bf16 MFMA: 1.6 times rocBLAS sgemm's speed at T = 3913.  Laid out
 // once, since splitting W in the GEMM would repeat it for every token group, and a pass per call would move ten bytes
-// per weight (90 us beside 126 us of GEMMs per 1.7B layer at T = 156).  Without the memory the prompts keep sgemm.
+// per weight (90 us beside 126 us of GEMMs per 1.7B layer at T = 156).  They are an option: made after everything the
+// decoder cannot do without, only while as much memory again stays free, given back when a later allocation fails
+// (drop_prompt_copies), and not made at all with QA_PROMPT_COPIES=0 (a decoder that runs no prompts, or whose memory is
+// wanted elsewhere); the prompts then run on sgemm.
 int pack_weights_prompt(qa_decoder * d) {
     if (d->layers.empty() || d->layers[0].qkv16 || !prompt_shapes(d)) return QA_OK;
+    const char * e = std::getenv("QA_PROMPT_COPIES");
+    if (e && std::strcmp(e, "0") == 0) return QA_OK;
     const qa_text_config & c = d->cfg;
     const int32_t H = c.hidden, QD = c.n_heads * kHeadDim, KD = c.n_kv_heads * kHeadDim, I = c.intermediate;
-    std::vector<void *> allocs;
+    const size_t elems = prompt_frag_elems(QD + 2 * KD, H) + prompt_frag_elems(H, QD) + prompt_frag_elems(2 * I, H) +
+                         prompt_frag_elems(H, I);
+    size_t free_bytes = 0, total_bytes = 0;
+    if (hipMemGetInfo(&free_bytes, &total_bytes) != hipSuccess ||
+        free_bytes < 2 * d->layers.size() * elems * sizeof(uint16_t)) {
+        (void)hipGetLastError();
+        return QA_OK;
+    }
     int rc = QA_OK;
     auto pack = [&](const float * src, int32_t N, int32_t K, uint16_t ** dst) {
         if (rc != QA_OK) return;
-        rc = dmalloc_t(allocs, prompt_frag_elems(N, K), dst);
+        rc = dmalloc_t(d->prompt_allocs, prompt_frag_elems(N, K), dst);
         if (rc == QA_OK) rc = prompt_split_launch(src, N, K, *dst, d->stream);
     };
     for (DevLayer & L : d->layers) {
@@ -681,13 +713,9 @@ int pack_weights_prompt(qa_decoder * d) {
         pack(L.down, H, I, &L.down3);
     }
     if (rc == QA_ERR_ALLOC) {
-        (void)hipGetLastError();
-        (void)hipStreamSynchronize(d->stream);
-        for (void * p : allocs) (void)hipFree(p);
-        for (DevLayer & L : d->layers) L.qkv3 = L.o3 = L.gu3 = L.down3 = nullptr;
+        (void)drop_prompt_copies(d);
         return QA_OK;
     }
-    d->weight_allocs.insert(d->weight_allocs.end(), allocs.begin(), allocs.end());
     return rc;
 }
 
@@ -811,7 +839,6 @@ extern "C" int qa_decoder_create(const qa_text_config * cfg, const qa_model_weig
     if (rc != QA_OK) return bail(rc);
     rc = pack_weights_bf16(d);
     if (rc == QA_OK) rc = pack_weights_mfma(d);
-    if (rc == QA_OK) rc = pack_weights_prompt(d);
     if (rc != QA_OK) return bail(rc);
 
     d->layout.n_layers = cfg->n_layers;
@@ -845,7 +872,8 @@ extern "C" int qa_decoder_create(const qa_text_config * cfg, const qa_model_weig
         hipMemsetAsync(d->am_ws, 0, d->am_ws_bytes, d->stream) != hipSuccess) {
         return bail(fail(QA_ERR_DEVICE, "workspace clear failed"));
     }
-    rc = ensure_rows(d, n_streams);
+    rc = pack_weights_prompt(d);
+    if (rc == QA_OK) rc = ensure_rows(d, n_streams);
     if (rc != QA_OK) return bail(rc);
     // QA_DECODE_PERSISTENT=1: the persistent decode step for callers that cannot call qa_decoder_set_persistent
     // (the drop-in API and its tools); a decoder it does not cover stays eager
@@ -866,6 +894,7 @@ extern "C" void qa_decoder_destroy(qa_decoder * d) {
     free_acts(d);
     for (void * p : d->weight_allocs) (void)hipFree(p);
     for (void * p : d->b16_allocs) (void)hipFree(p);
+    for (void * p : d->prompt_allocs) (void)hipFree(p);
     if (d->staging) (void)hipFree(d->staging);
     if (d->cache) (void)hipFree(d->cache);
     if (d->h_ids) (void)hipHostFree(d->h_ids);
@@ -1026,12 +1055,9 @@ extern "C" int qa_decoder_decode_streams(qa_decoder * d, const int32_t * first_i
     return QA_OK;
 }
 
-extern "C" int qa_decoder_set_persistent(qa_decoder * d, int32_t enable) {
-    if (!d) return fail(QA_ERR_INVALID, "qa_decoder_set_persistent: null decoder");
-    if (!enable) {
-        d->persist = false;
-        return QA_OK;
-    }
+namespace {
+
+int enable_persistent(qa_decoder * d) {
     int32_t grid = 0;
     int rc = persist_plan(persist_plan_in(d), &grid);
     if (rc != QA_OK) return rc;
@@ -1088,6 +1114,18 @@ extern "C" int qa_decoder_set_persistent(qa_decoder * d, int32_t enable) {
     return QA_OK;
 }
 
+}  // namespace
+
+extern "C" int qa_decoder_set_persistent(qa_decoder * d, int32_t enable) {
+    if (!d) return fail(QA_ERR_INVALID, "qa_decoder_set_persistent: null decoder");
+    if (!enable) {
+        d->persist = false;
+        return QA_OK;
+    }
+    const int rc = enable_persistent(d);
+    return rc == QA_ERR_ALLOC && drop_prompt_copies(d) ? enable_persistent(d) : rc;
+}
+
 extern "C" int qa_decoder_fill_cache(qa_decoder * d, int32_t stream, const float * k, const float * v, int32_t len) {
     if (!d || !k || !v || stream < 0 || stream >= d->n_streams || len < 0 || len > d->max_seq) {
         return fail(QA_ERR_INVALID, "qa_decoder_fill_cache: invalid arguments");
@@ -1098,7 +1136,9 @@ extern "C" int qa_decoder_fill_cache(qa_decoder * d, int32_t stream, const float
         if (d->staging) (void)hipFree(d->staging);
         d->staging = nullptr;
         d->staging_bytes = 0;
-        if (hipMalloc(reinterpret_cast<void **>(&d->staging), per_layer * sizeof(float)) != hipSuccess) {
+        if (hipMalloc(reinterpret_cast<void **>(&d->staging), per_layer * sizeof(float)) != hipSuccess &&
+            !(drop_prompt_copies(d) &&
+              hipMalloc(reinterpret_cast<void **>(&d->staging), per_layer * sizeof(float)) == hipSuccess)) {
             return fail(QA_ERR_ALLOC, "staging allocation failed");
         }
         d->staging_bytes = per_layer * sizeof(float);
