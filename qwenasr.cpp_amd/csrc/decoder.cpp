@@ -215,6 +215,13 @@ bool prompt_ready(const qa_decoder * d) {
     return !d->layers.empty() && (d->layers[0].qkv16 || d->layers[0].qkv3) && prompt_shapes(d);
 }
 
+// Fewest rows that take them.  f32 weights up to 32 rows keep the skinny f32 GEMM: it reads 4 instead of 6 bytes per
+// weight, and one 32-row pass is as fast or faster (whole calls of 4 layers, us, sgemm path / prompt GEMM: 0.6B 2 rows
+// 429 / 464, 20 rows 464 / 484, 32 rows 488 / 495, 33 rows 611 / 497; 1.7B 672 / 700, 710 / 728, 736 / 746, 1034 / 745).
+int32_t prompt_min_rows(const qa_decoder * d) {
+    return !prompt_ready(d) ? INT32_MAX : d->layers[0].qkv16 ? 2 : 33;
+}
+
 // Gives the prompt copies of f32 weights back after an allocation failed; the activations are laid out again by the
 // next ensure_rows (prompts then run on sgemm, which needs other buffers).
 bool drop_prompt_copies(qa_decoder * d) {
@@ -240,7 +247,8 @@ int alloc_rows(qa_decoder * d, int32_t rows) {
     rc = rc ? rc : dmalloc_t(d->act_allocs, R * (QD + 2 * KD), &d->qkv);
     rc = rc ? rc : dmalloc_t(d->act_allocs, R * QD, &d->qrot);
     rc = rc ? rc : dmalloc_t(d->act_allocs, R * QD, &d->attn);
-    if (!prompt_ready(d)) rc = rc ? rc : dmalloc_t(d->act_allocs, R * 2 * I, &d->gu);
+    const size_t gu_rows = std::min(rows, prompt_min_rows(d) - 1);   // rows that do not run the prompt GEMMs
+    if (gu_rows >= 2) rc = rc ? rc : dmalloc_t(d->act_allocs, gu_rows * 2 * I, &d->gu);
     rc = rc ? rc : dmalloc_t(d->act_allocs, R * I, &d->act);
     // the LM head runs on one row per stream (decode) or the last row (prefill)
     const size_t gr = rows >= 2 ? gemm_rows_bytes_for(d->cfg, std::min<int32_t>(rows, kSkinnyRows),
@@ -260,7 +268,7 @@ int alloc_rows(qa_decoder * d, int32_t rows) {
         const size_t n = static_cast<size_t>((H + 15) / 16) * 32;
         rc = dmalloc(d->act_allocs, n * sizeof(double), reinterpret_cast<void **>(&d->xstats));
     }
-    if (rc == QA_OK && rows >= 2 && prompt_ready(d)) {
+    if (rc == QA_OK && rows >= prompt_min_rows(d)) {
         d->partial_bytes = prompt_partial_bytes(rows);
         rc = dmalloc_t(d->act_allocs, prompt_frag_elems(rows, std::max(d->cfg.hidden, d->cfg.n_heads * kHeadDim)), &d->xf);
         rc = rc ? rc : dmalloc_t(d->act_allocs, prompt_frag_elems(rows, d->cfg.intermediate), &d->actf);
@@ -378,7 +386,7 @@ int run_layer(qa_decoder * d, int32_t l, int32_t rows, int kind, int32_t n_past,
     const int32_t H = c.hidden, QD = c.n_heads * kHeadDim, KD = c.n_kv_heads * kHeadDim, I = c.intermediate;
     const int32_t W3 = QD + 2 * KD;
     hipStream_t s = d->stream;
-    const bool prompt = rows > 1 && !fused && d->xf;
+    const bool prompt = !fused && d->xf && rows >= prompt_min_rows(d);
     int32_t slices = 0;        // K slices of the q|k|v projection, still partial sums in d->partial
     bool attn_split = false;   // the attention left its output split in d->xf
     int rc;

@@ -52,7 +52,8 @@ def test_layer_matches_oracle(qa, orc, bf16, cached):
 @pytest.mark.parametrize("T", [2, 33, 100, 156, 300, 640, 1037, 2100])
 def test_three_part_weights_equal_bf16_copies(qa, T):
     """f32 weights that hold bf16 values: their mid and lo parts add exact zeros, so the three-part GEMM gives the
-    bits of the GEMM on the bf16 copies, whatever the plan (2100 rows: 256 columns per workgroup against 128)."""
+    bits of the GEMM on the bf16 copies, whatever the plan (2100 rows: 256 columns per workgroup against 128).  Up to 32
+    rows f32 weights do not run it."""
     model = qa.Model(qa.QWEN3_ASR_0_6B, n_layers=1, bf16=True)
     x = qa.prompt_input(model, T - 1, 1)
     out = []
@@ -61,4 +62,27 @@ def test_three_part_weights_equal_bf16_copies(qa, T):
             assert dec.weights_bf16 == (not f32_weights)
             out.append(dec.layer_forward(0, x, 0))
     assert np.isfinite(out[0]).all()
+    if T <= 32:   # the skinny f32 GEMM: another order of the same sums, as above
+        d = out[1].astype(np.float64) - out[0]
+        assert np.linalg.norm(d) <= 1.4e-5 * np.linalg.norm(out[0])
+        return
     np.testing.assert_array_equal(out[0].view(np.uint32), out[1].view(np.uint32))
+
+
+@pytest.mark.parametrize("T", [2, 17, 32, 33])
+def test_f32_weights_up_to_32_rows_read_the_f32_weights(qa, T):
+    """Up to 32 positions the f32 rows are the shorter read (4 bytes per weight against 6): the copies change no bit."""
+    model = qa.Model(qa.QWEN3_ASR_0_6B, n_layers=1)
+    x = qa.prompt_input(model, T - 1, 1)
+    out = []
+    for copies in ("1", "0"):
+        os.environ["QA_PROMPT_COPIES"] = copies
+        try:
+            with qa.Decoder(model, 1, 300, qa.QA_CACHE_F32) as dec:
+                dec.layer_forward(0, qa.prompt_input(model, 299, 1), 0)    # activations for longer prompts too
+                out.append(dec.layer_forward(0, x, 0))
+        finally:
+            del os.environ["QA_PROMPT_COPIES"]
+    assert np.array_equal(out[0].view(np.uint32), out[1].view(np.uint32)) == (T <= 32)
+    d = out[1].astype(np.float64) - out[0]
+    assert np.linalg.norm(d) <= 1.4e-5 * np.linalg.norm(out[0])
