@@ -23,11 +23,14 @@ __device__ inline void store_split3(uint16_t * o, int64_t K, float v) {
     o[2 * K] = static_cast<uint16_t>(__float_as_uint(r2) >> 16);
 }
 
-// the three parts of v as bf16 bits (an infinity: itself, 0, 0, so that its products are those of an f32 GEMM)
+// the three parts of v as bf16 bits.  An infinity is 0, 0, itself: the last part meets only the leading part of the
+// other operand, which is zero for a zero alone, so its products are those of an f32 GEMM (as the leading part it would
+// meet parts that are zero, and infinity times zero is NaN).
 __device__ inline void split3_parts(float v, uint16_t & hi, uint16_t & mid, uint16_t & lo) {
-    const uint32_t h = __float_as_uint(v) & 0xffff0000u;
-    const float r1 = v == __uint_as_float(h) ? 0.0f : v - __uint_as_float(h);
-    const uint32_t m = __float_as_uint(r1) & 0xffff0000u;
+    const bool inf = __builtin_isinf(v);
+    const uint32_t h = inf ? 0u : __float_as_uint(v) & 0xffff0000u;
+    const float r1 = v - __uint_as_float(h);
+    const uint32_t m = inf ? 0u : __float_as_uint(r1) & 0xffff0000u;
     hi = static_cast<uint16_t>(h >> 16);
     mid = static_cast<uint16_t>(m >> 16);
     lo = static_cast<uint16_t>(__float_as_uint(r1 - __uint_as_float(m)) >> 16);
