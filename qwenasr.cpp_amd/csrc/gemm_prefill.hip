@@ -6,8 +6,8 @@
 // MFMAs: f32 products and f32 sums, as the reference's GEMM, in another order.
 //   bf16-exact weights (WP 1, one part):  lo w, mid w, hi w                              3 MFMAs per 16 k
 //   f32 weights (WP 3, three parts):      lo hi, hi lo, mid mid, mid hi, hi mid, hi hi   6 MFMAs per 16 k
-// The products left out of the second form (mid lo, lo mid, lo lo) are below 2^-24 of the whole one, under the
-// rounding of one f32 sum.  Relative error against float64 (2-norm, N(0, 1) rows, 1.7B shapes): 7.0e-7 at K = 2048
+// The products left out of the second form (mid lo, lo mid, lo lo) are within 2^-24 of the whole one, the rounding of
+// one f32 sum, and of either sign, since hi and mid are rounded to nearest (split3.hpp).  Relative error against float64 (2-norm, N(0, 1) rows, 1.7B shapes): 7.0e-7 at K = 2048
 // and 1.3e-6 at K = 6144 with one K slice, 2-5e-7 with several; rocBLAS sgemm 8.1e-7 and 1.0-1.4e-6.  Parts that
 // are zero add exact zeros, and both forms follow one plan and one order, so f32 weights that hold bf16 values give
 // the bits of their bf16 copies.

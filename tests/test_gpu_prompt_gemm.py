@@ -30,8 +30,9 @@ def _decoder(qa, model, max_seq, f32_weights):
 @pytest.mark.parametrize("bf16", [False, True], ids=["f32-weights", "bf16-copies"])
 @pytest.mark.parametrize("cached", [False, True], ids=["nocache", "cached"])
 def test_layer_matches_oracle(qa, orc, bf16, cached):
-    """Four projections in sequence, each a sum of at most 3072 exact products: two orders of an f32 sum of n terms
-    differ by about sqrt(n) 2^-24 = 3.3e-6 of the result, so a layer by at most 1.4e-5 (relative 2-norm)."""
+    """Four projections in sequence, each a sum of at most 3072 products (exact, or within 2^-24 on f32 weights): two orders
+    of an f32 sum of n terms differ by about sqrt(n) 2^-24 = 3.3e-6 of the result, so a layer by at most 1.4e-5
+    (relative 2-norm)."""
     model = qa.Model(qa.QWEN3_ASR_0_6B, n_layers=1, bf16=bf16)
     om = orc.OracleModel.from_product_model(model)
     x = qa.prompt_input(model, max(LENGTHS) - 10, 10)

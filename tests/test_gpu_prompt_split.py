@@ -39,3 +39,56 @@ def test_infinite_input_keeps_the_sign_of_its_weight(qa, T, bf16):
     want = np.broadcast_to(np.copysign(np.float32(np.inf), down[:, 5]), got.shape)
     assert (down[:, 5] != 0).all()
     np.testing.assert_array_equal(got, want)
+
+
+def _cached_v(qa, dec, T):
+    """V rows [T][1024] of layer 0 of a decoder's f32 cache."""
+    address, lay = dec.cache()
+    host = np.empty((2, lay.n_kv_heads, lay.max_seq, 128), np.float32)
+    qa.check(qa.lib.qa_copy_to_host(host.ctypes.data, address, host.nbytes))
+    return host[1, :, :T].transpose(1, 0, 2).reshape(T, -1)
+
+
+@pytest.mark.parametrize("size", ["0.6B", "1.7B"])
+@pytest.mark.parametrize("T", [33, 64, 96, 130, 156, 200, 300, 1100])
+def test_single_products_of_f32_weights(qa, size, T):
+    """One weight per row of v, so that each output is one product of six part products: what is left out is at most
+    2^-24 of it, and the sums round once by at most 2^-23 (a sum of parts that is below 2^-7 of the whole adds less than a
+    tenth of that).  Mantissas are those whose parts are largest beside random ones; a part product that is missing is
+    2^-16 of the result."""
+    z = {"0.6B": qa.QWEN3_ASR_0_6B, "1.7B": qa.QWEN3_ASR_1_7B}[size]
+    model = qa.Model(z, n_layers=1, vocab=4096)
+    rng = np.random.default_rng(T)
+
+    def values(n):
+        low = rng.choice(np.array([0xFFFF, 0x7FFF, 0x8000, 0x8001, 0x0001, 0xFF7F, 0x0080, 0xFF80], np.uint32), n)
+        low = np.where(rng.random(n) < 0.3, rng.integers(0, 1 << 16, n, dtype=np.uint32), low)
+        top = np.where(rng.random(n) < 0.5, 0, rng.integers(0, 128, n)).astype(np.uint32)
+        exponent = rng.integers(124, 131, n, dtype=np.uint32)
+        return (rng.integers(0, 2, n, dtype=np.uint32) << 31 | exponent << 23 | top << 16 | low).view(np.float32)
+
+    at = np.arange(1024) * (z.hidden // 1024) + np.arange(1024) % (z.hidden // 1024)
+    w = values(1024)
+    # past the largest bf16, where rounding would give infinity
+    w[:4] = np.array([0x7F7FFFFF, 0xFF7FFFFF, 0x7F7F8000, 0x7F7F7FFF], np.uint32).view(np.float32)
+    wv = _tensor(model, "attn_v")
+    wv[:] = 0.0
+    wv[np.arange(1024), at] = w
+    nw = values(z.hidden)
+    nw[at[:4]] *= np.float32(2.0 ** -20)
+    model.tensor("text.blk.0.attn_norm.weight")[:] = nw
+    x = rng.choice(np.array([-1.0, 1.0], np.float32), (T, z.hidden))
+    # the RMSNorm of rows of ones: mean square 1, float scale, (x scale) w
+    scale = np.float32(1.0) / np.sqrt(np.float32(1.0) + np.float32(model.cfg.rms_norm_eps))
+    xn = (x * scale).astype(np.float32) * nw
+    print(f"single products {size} T={T}", flush=True)
+    with qa.Decoder(model, 1, T, qa.QA_CACHE_F32) as dec:
+        assert not dec.weights_bf16
+        dec.layer_forward(0, x, 0)
+        got = _cached_v(qa, dec, T)
+    want = xn[:, at].astype(np.float64) * w
+    off = np.abs(got - want) / np.abs(want) * 2.0 ** 24
+    print(f"  largest error {off.max():.2f} x 2^-24, mean of the signed error towards zero "
+          f"{((np.abs(want) - np.abs(got)) / np.abs(want)).mean() * 2.0 ** 24:.3f} x 2^-24", flush=True)
+    assert off.max() <= 3.2
+
