@@ -712,7 +712,7 @@ int pack_weights_prompt(qa_decoder * d) {
     auto pack = [&](const float * src, int32_t N, int32_t K, uint16_t ** dst) {
         if (rc != QA_OK) return;
         rc = dmalloc_t(d->prompt_allocs, prompt_frag_elems(N, K), dst);
-        if (rc == QA_OK) rc = prompt_split_launch(src, N, K, *dst, d->stream);
+        if (rc == QA_OK) rc = prompt_pack_launch(src, N, K, *dst, d->stream);
     };
     for (DevLayer & L : d->layers) {
         pack(L.qkv, QD + 2 * KD, H, &L.qkv3);

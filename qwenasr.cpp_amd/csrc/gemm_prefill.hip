@@ -7,10 +7,18 @@
 //   bf16-exact weights (WP 1, one part):  lo w, mid w, hi w                              3 MFMAs per 16 k
 //   f32 weights (WP 3, three parts):      lo hi, hi lo, mid mid, mid hi, hi mid, hi hi   6 MFMAs per 16 k
 // The products left out of the second form (mid lo, lo mid, lo lo) are within 2^-24 of the whole one, the rounding of
-// one f32 sum, and of either sign, since hi and mid are rounded to nearest (split3.hpp).  Relative error against float64 (2-norm, N(0, 1) rows, 1.7B shapes): 7.0e-7 at K = 2048
-// and 1.3e-6 at K = 6144 with one K slice, 2-5e-7 with several; rocBLAS sgemm 8.1e-7 and 1.0-1.4e-6.  Parts that
-// are zero add exact zeros, and both forms follow one plan and one order, so f32 weights that hold bf16 values give
-// the bits of their bf16 copies.
+// one f32 sum, and of either sign, since hi and mid are rounded to nearest (split3.hpp).  Parts that are zero add exact
+// zeros, and both forms follow one plan and one order, so f32 weights that hold bf16 values give the bits of their bf16
+// copies.
+//
+// Sums.  The bf16 MFMA rounds its sums down a little more often than up (a mean of 2 to 10% of a last place, whatever the
+// sign), and six MFMAs per 16 k on f32 weights add up to -1.1e-7 of the outputs' root mean square over 2048 k: the same
+// for every token, so an average over tokens, as the attention takes, keeps it while it loses the signal.  X is therefore
+// stored negated in every second pair of blocks of 256 k (split_negated), and the accumulators turn round with it: 1e-9.
+// Up to 64 tokens (SUMS) every block of 256 k is a sum of its own, as short as the chains of the f32 kernel before.
+// Relative error against float64 (2-norm, N(0, 1) rows): q|k|v of 2048 k 1.9e-7 at 33 to 64 tokens (gemm_rows_kernel
+// 2.0-2.2e-7), 3.5e-7 at 156 and 6.9e-7 from 700 on (sgemm 8.1e-7); a 1.7B layer whose residual is scaled away 0.72-0.77e-6
+// (0.77-0.79e-6), 1.5e-6 at 156 and 2.3-2.6e-6 from 700 on (sgemm 2.8-3.0e-6; without the negation 2.9-4.2e-6).
 //
 // Layout.  X comes in MFMA fragment order (frag offset in split3.hpp): the operand of one MFMA, 32 rows x 16 k of
 // one part, is 1 KB of consecutive memory, so a wave loads it from L2 straight into the operand registers with one
@@ -50,7 +58,7 @@ constexpr int kPgMaxSplitWgs = 320;        // workgroups of a plan with K slices
 
 struct PgParams {
     const uint16_t * Xf;     // fragment-ordered split of X (frag_index)
-    const uint16_t * W;      // WP 1: [rows of W][K] bf16 bits; WP 3: fragment-ordered split of W (prompt_pack)
+    const uint16_t * W;      // WP 1: [rows of W][K] bf16 bits; WP 3: fragment-ordered split of W (prompt_pack_launch)
     float * Y;               // [M][N] (store, accumulate) or the partials [ks][M][N]
     uint16_t * act;          // SwiGLU: fragment-ordered split of silu(gate) * up, [M][N]
     int32_t M, N, K;         // N output columns (SwiGLU: W has 2 N rows)
@@ -68,9 +76,10 @@ struct Stage {
     static constexpr int kBlocks = WP == 1 ? 4 * NT : kSteps * 3 * NT;   // 1 KB each
 };
 
-// NT: MFMA tiles of 32 columns per wave.  LPW: 1 KB blocks of a W stage that each wave loads, ceil(kBlocks / wm)
-template <int WP, int EPI, int NT, int LPW>
-__global__ __launch_bounds__(64 * kMaxWaves) void gemm_prefill_kernel(PgParams p) {
+// NT: MFMA tiles of 32 columns per wave.  LPW: 1 KB blocks of a W stage that each wave loads, ceil(kBlocks / wm).
+// SUMS: at most four waves per workgroup, which leaves each the registers for a second set of accumulators
+template <int WP, int EPI, int NT, int LPW, bool SUMS>
+__global__ __launch_bounds__(64 * (SUMS ? 4 : kMaxWaves)) void gemm_prefill_kernel(PgParams p) {
 #pragma clang fp contract(off)
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
     using St = Stage<WP, NT>;
@@ -220,15 +229,46 @@ __global__ __launch_bounds__(64 * kMaxWaves) void gemm_prefill_kernel(PgParams p
     for (int b = 0; b < SK; ++b) load_x(0, b);
     __builtin_amdgcn_sched_barrier(0);
     write_w(0);
-    for (int s = 0; s < my; ++s) {
-        __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): this wave's part of stage s is in LDS
-        __builtin_amdgcn_s_barrier();          // and every wave's; nobody reads stage s - 1 any more
-        __builtin_amdgcn_sched_barrier(0);
-        load_w(s + 1);
-        __builtin_amdgcn_sched_barrier(0);
-        compute(ring + (s & 1) * kStageBytes, s);
-        write_w(s + 1);
-        __builtin_amdgcn_sched_barrier(0);
+    // stages in parts of at most kSplitSign k.  Where the sign of X changes the accumulators turn round with it; SUMS: each
+    // part is added to a sum of its own and the accumulators start again (see the header)
+    constexpr int kPart = kSplitSign / (16 * SK);
+    v16f sums[SUMS ? NT : 1];
+    if constexpr (SUMS) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) sums[j] = v16f{};
+    }
+    for (int s = 0; s < my;) {
+        const int end = min(my, s + kPart - (s0 + s) % kPart);
+        const bool minus = split_negated((s0 + s) * 16 * SK);
+        for (; s < end; ++s) {
+            __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): this wave's part of stage s is in LDS
+            __builtin_amdgcn_s_barrier();          // and every wave's; nobody reads stage s - 1 any more
+            __builtin_amdgcn_sched_barrier(0);
+            load_w(s + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            compute(ring + (s & 1) * kStageBytes, s);
+            write_w(s + 1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (SUMS) {
+            const float sign = minus ? -1.0f : 1.0f;
+            if (s < my) {
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) sums[j][e] = __builtin_fmaf(sign, acc[j][e], sums[j][e]);
+                    acc[j] = v16f{};
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) acc[j][e] = __builtin_fmaf(sign, acc[j][e], sums[j][e]);
+            }
+        } else if (s < my ? minus != split_negated((s0 + s) * 16 * SK) : minus) {
+#pragma unroll
+            for (int j = 0; j < NT; ++j) acc[j] = -acc[j];
+        }
     }
     // the K groups of the workgroup, in order, through LDS
     if (p.kw > 1) {
@@ -390,12 +430,12 @@ __global__ __launch_bounds__(R == 1 ? 256 : 512) void prompt_norm_kernel(float *
         float y[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) y[e] = v[i][e] * scale * nw[i][e];
-        store_frag8(Xf, dim / 16, static_cast<int>(r), o, y);
+        store_frag8<true>(Xf, dim / 16, static_cast<int>(r), o, y);
     }
 }
 
 // Thread = 8 consecutive values of one row; consecutive threads take 8 neighbouring rows, whose pieces of a fragment
-// fill whole lines.  MODE 0: the split of src; 1: the split of silu(gate) up over the partial sums [ks][rows][2 dim]
+// fill whole lines.  MODE 0: the split of src (3: of weights, without the signs of an input); 1: the split of silu(gate) up over the partial sums [ks][rows][2 dim]
 // (rows gate | up); 2: the sum of the partial sums, stored to dst.
 template <int MODE>
 __global__ __launch_bounds__(256) void prompt_rows_kernel(const float * src, int ks, int rows, int dim, float * dst,
@@ -409,7 +449,7 @@ __global__ __launch_bounds__(256) void prompt_rows_kernel(const float * src, int
     const int o = static_cast<int>(i8 - rb * oct);
     if (r >= rows) return;
     float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if constexpr (MODE == 0) {
+    if constexpr (MODE == 0 || MODE == 3) {
         load8(src + r * dim + o * 8, v);
     } else if constexpr (MODE == 1) {
         float u[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -422,7 +462,7 @@ __global__ __launch_bounds__(256) void prompt_rows_kernel(const float * src, int
         store8(dst + r * dim + o * 8, v);
         return;
     }
-    store_frag8(Xf, dim / 16, static_cast<int>(r), o, v);
+    store_frag8<MODE != 3>(Xf, dim / 16, static_cast<int>(r), o, v);
 }
 
 template <int MODE>
@@ -485,15 +525,15 @@ Plan prompt_plan(int32_t M, int64_t cols, int32_t units, bool swiglu) {
     return best;
 }
 
-template <int WP, int EPI, int NT, int LPW>
+template <int WP, int EPI, int NT, int LPW, bool SUMS = false>
 int launch_one(const PgParams & p, hipStream_t stream) {
     const size_t lds = std::max(static_cast<size_t>(p.kw) * 2 * Stage<WP, NT>::kBlocks * 1024,
                                 static_cast<size_t>(p.kw - 1) * p.wm * NT * 1024 * sizeof(float));
     if (lds > 64 * 1024) {
-        QA_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_prefill_kernel<WP, EPI, NT, LPW>),
+        QA_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_prefill_kernel<WP, EPI, NT, LPW, SUMS>),
                                    hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
     }
-    hipLaunchKernelGGL((gemm_prefill_kernel<WP, EPI, NT, LPW>), dim3(static_cast<unsigned>(p.m_groups * p.n_groups * p.ks)),
+    hipLaunchKernelGGL((gemm_prefill_kernel<WP, EPI, NT, LPW, SUMS>), dim3(static_cast<unsigned>(p.m_groups * p.n_groups * p.ks)),
                        dim3(static_cast<unsigned>(64 * p.wm * p.kw)), lds, stream, p);
     QA_LAUNCH_CHECK("gemm_prefill_kernel");
     return QA_OK;
@@ -506,7 +546,11 @@ int launch_wm(const PgParams & p, int nt, hipStream_t stream) {
         if (nt == 8) return launch_one<WP, EPI, 8, 4>(p, stream);
     }
     switch (p.wm) {
-        case 2: return launch_one<WP, EPI, 4, B / 2>(p, stream);
+        case 2:
+            // the sums of short blocks for up to 64 tokens, where f32 weights had sums as short before; with more groups of
+            // tokens one workgroup per CU, as their registers ask for, costs more than it brings (f32 weights, whole calls
+            // of 4 layers: 100 tokens 899 / 912 us, 300 tokens 1451 / 1483)
+            return p.m_groups == 1 ? launch_one<WP, EPI, 4, B / 2, true>(p, stream) : launch_one<WP, EPI, 4, B / 2>(p, stream);
         case 3: return launch_one<WP, EPI, 4, (B + 2) / 3>(p, stream);
         case 4: return launch_one<WP, EPI, 4, B / 4>(p, stream);
         case 5: return launch_one<WP, EPI, 4, (B + 4) / 5>(p, stream);
@@ -598,6 +642,10 @@ int prompt_norm_launch(float * x, const float * partial, int32_t slices, const f
 
 int prompt_split_launch(const float * x, int32_t rows, int32_t dim, uint16_t * Xf, hipStream_t stream) {
     return launch_rows<0>(x, 0, rows, dim, nullptr, Xf, stream);
+}
+
+int prompt_pack_launch(const float * w, int32_t rows, int32_t dim, uint16_t * Wf, hipStream_t stream) {
+    return launch_rows<3>(w, 0, rows, dim, nullptr, Wf, stream);
 }
 
 int prompt_swiglu_launch(const float * partial, int32_t slices, int32_t rows, int32_t dim, uint16_t * Xf,

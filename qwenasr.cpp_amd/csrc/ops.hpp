@@ -12,7 +12,7 @@ int gemv_launch(int epi, bool prenorm, const float * W, int32_t out_dim, int32_t
                 const float * norm_w, float eps, hipStream_t stream, const uint16_t * W16 = nullptr);
 // Prompt projections (gemm_prefill.hip): Y[M][N] (+)= X[M][K] W[N][K]^T, X given as its fragment-ordered three-part
 // split (prompt_frag_elems bf16 values), W as the bf16 bits of bf16-exact weights (W16) or as the same split of f32
-// weights (W3, prompt_split_launch of their rows); with act != nullptr W = [gate rows; up rows]
+// weights (W3, prompt_pack_launch of their rows); with act != nullptr W = [gate rows; up rows]
 // (2 N rows) and act receives the fragment-ordered split of silu(gate) * up.  *slices = 0: done; otherwise the
 // *slices K slices' partial sums [slices][M][W rows] lie in `partial` and the next row kernel adds them up.
 struct PromptGemm {
@@ -34,6 +34,7 @@ int prompt_gemm_launch(const PromptGemm & g, int32_t * slices, hipStream_t strea
 int prompt_norm_launch(float * x, const float * partial, int32_t slices, const float * w, int32_t rows, int32_t dim,
                        float eps, uint16_t * Xf, hipStream_t stream);
 int prompt_split_launch(const float * x, int32_t rows, int32_t dim, uint16_t * Xf, hipStream_t stream);
+int prompt_pack_launch(const float * w, int32_t rows, int32_t dim, uint16_t * Wf, hipStream_t stream);
 // Xf = the split of silu(gate) up, gate | up summed over partial [slices][rows][2 dim]
 int prompt_swiglu_launch(const float * partial, int32_t slices, int32_t rows, int32_t dim, uint16_t * Xf,
                          hipStream_t stream);

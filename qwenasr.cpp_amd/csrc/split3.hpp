@@ -46,28 +46,36 @@ __device__ inline void split3_pair(float a, float b, uint32_t & hi, uint32_t & m
     lo = pack(a - low(mid), b - high(mid));
 }
 
+// Inputs of the prompt GEMM are stored negated where this holds, in blocks + - - + of kSplitSign k (gemm_prefill.hip says
+// what for).
+constexpr int kSplitSign = 256;
+__device__ inline bool split_negated(int k) { return ((k / kSplitSign ^ k / (2 * kSplitSign)) & 1) != 0; }
+
 // 8 consecutive k (octet o) of row r into the fragment order of an MFMA operand: 32 rows x 16 k of one part are
 // 512 consecutive values, lane l = row % 32 + 32 (k / 8 % 2) holding k % 8 = 0..7; fragments follow each other by
-// part (hi, mid, lo), then k / 16, then row / 32.
+// part (hi, mid, lo), then k / 16, then row / 32.  INPUT: negated where split_negated.
+template <bool INPUT>
 __device__ inline void store_frag8(uint16_t * out, int k16, int r, int o, const float (&v)[8]) {
+    const uint32_t sign = INPUT && split_negated(8 * o) ? 0x80008000u : 0u;
     uint32_t part[3][4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) split3_pair(v[2 * e], v[2 * e + 1], part[0][e], part[1][e], part[2][e]);
     uint16_t * d = out + (static_cast<int64_t>(r >> 5) * k16 + (o >> 1)) * 3 * 512 + ((r & 31) + 32 * (o & 1)) * 8;
 #pragma unroll
     for (int w = 0; w < 3; ++w) {
-        *reinterpret_cast<uint4 *>(d + w * 512) = make_uint4(part[w][0], part[w][1], part[w][2], part[w][3]);
+        *reinterpret_cast<uint4 *>(d + w * 512) = make_uint4(part[w][0] ^ sign, part[w][1] ^ sign, part[w][2] ^ sign, part[w][3] ^ sign);
     }
 }
 
-// 4 consecutive k (first k % 4 == 0) of row r into the same order
+// 4 consecutive k (first k % 4 == 0) of row r of an input into the same order
 __device__ inline void store_frag4(uint16_t * out, int k16, int r, int k, float v0, float v1, float v2, float v3) {
+    const uint32_t sign = split_negated(k) ? 0x80008000u : 0u;
     uint32_t part[3][2];
     split3_pair(v0, v1, part[0][0], part[1][0], part[2][0]);
     split3_pair(v2, v3, part[0][1], part[1][1], part[2][1]);
     uint16_t * d = out + (static_cast<int64_t>(r >> 5) * k16 + (k >> 4)) * 3 * 512 + ((r & 31) + 32 * ((k >> 3) & 1)) * 8 + (k & 7);
 #pragma unroll
-    for (int w = 0; w < 3; ++w) *reinterpret_cast<uint2 *>(d + w * 512) = make_uint2(part[w][0], part[w][1]);
+    for (int w = 0; w < 3; ++w) *reinterpret_cast<uint2 *>(d + w * 512) = make_uint2(part[w][0] ^ sign, part[w][1] ^ sign);
 }
 
 }  // namespace qa

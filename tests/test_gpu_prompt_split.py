@@ -92,3 +92,58 @@ def test_single_products_of_f32_weights(qa, size, T):
           f"{((np.abs(want) - np.abs(got)) / np.abs(want)).mean() * 2.0 ** 24:.3f} x 2^-24", flush=True)
     assert off.max() <= 3.2
 
+
+def _layer64(model, x, T):
+    """The layer in 64 bits, from position 0 (text-decoder.cpp:265-345), and its v."""
+    H, eps, theta = model.cfg.hidden, model.cfg.rms_norm_eps, model.cfg.rope_theta
+    mat = lambda name: _tensor(model, name).astype(np.float64)
+    vec = lambda name: model.tensor(f"text.blk.0.{name}.weight").astype(np.float64)
+    rms = lambda a, w: a / np.sqrt(np.square(a).mean(-1, keepdims=True) + eps) * w
+    x = x.astype(np.float64)
+    h = rms(x, vec("attn_norm"))
+    angle = np.arange(T)[:, None] * theta ** (-np.arange(64) / 64.0)
+    c, s = np.cos(angle), np.sin(angle)
+
+    def rope(a):                                      # [heads, T, 128]
+        lo, hi = a[..., :64], a[..., 64:]
+        return np.concatenate([lo * c - hi * s, hi * c + lo * s], -1)
+
+    heads = lambda name: (h @ mat(name).T).reshape(T, -1, 128).transpose(1, 0, 2)
+    q, k, v = rope(rms(heads("attn_q"), vec("attn_q_norm"))), rope(rms(heads("attn_k"), vec("attn_k_norm"))), heads("attn_v")
+    out = np.empty((T, 2048))
+    for i in range(16):
+        sc = q[i] @ k[i // 2].T / np.sqrt(128.0)
+        sc[np.triu_indices(T, 1)] = -np.inf
+        p = np.exp(sc - sc.max(1, keepdims=True))
+        out[:, 128 * i:128 * i + 128] = p @ v[i // 2] / p.sum(1, keepdims=True)
+    x = x + out @ mat("attn_output").T
+    h = rms(x, vec("ffn_norm"))
+    g = h @ mat("ffn_gate").T
+    y = x + (g / (1.0 + np.exp(-g)) * (h @ mat("ffn_up").T)) @ mat("ffn_down").T
+    return y, v.transpose(1, 0, 2).reshape(T, -1)
+
+
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32-weights", "bf16-copies"])
+@pytest.mark.parametrize("size,T", [("0.6B", 40), ("0.6B", 156), ("1.7B", 52), ("1.7B", 156), ("1.7B", 300), ("1.7B", 700)])
+def test_layer_without_residual_against_64_bits(qa, size, T, bf16):
+    """o and down are scaled up, so that the residual is 1/100 of each sum and hides nothing.  The error is that of four
+    projections in a row: f32 sums over 2048 k are off by 0.7e-6 and over 6144 by 1.2e-6 at most, q|k|v, o, gate and up
+    (whose errors both go into down) and down together 2.0e-6, and a factor 1.3 for the seed.  A part product left out of
+    any one of them moves the output by 1.0e-5; rounding towards one side in the sums is an error that all tokens share,
+    which the attention's average over 700 tokens keeps (2.9e-6), and shows in the mean of v: 1e-7 of its root mean square
+    in every row, where independent errors leave less than 2e-9."""
+    z = {"0.6B": qa.QWEN3_ASR_0_6B, "1.7B": qa.QWEN3_ASR_1_7B}[size]
+    model = qa.Model(z, n_layers=1, vocab=4096, bf16=bf16)
+    _tensor(model, "attn_output")[:] *= 64.0
+    _tensor(model, "ffn_down")[:] *= 8192.0
+    x = qa.prompt_input(model, T - 1, 1)
+    print(f"layer {size} T={T} bf16={bf16}", flush=True)
+    with qa.Decoder(model, 1, T, qa.QA_CACHE_F32) as dec:
+        assert dec.weights_bf16 == bf16
+        got = dec.layer_forward(0, x, 0)
+        v = _cached_v(qa, dec, T)
+    want, want_v = _layer64(model, x, T)
+    bias = (v - want_v).mean() / np.sqrt(np.square(want_v).mean())
+    off = np.linalg.norm(got - want) / np.linalg.norm(want)
+    print(f"  {off:.2e}, mean of v {bias:.1e}", flush=True)
+    assert off <= 2.6e-6 and abs(bias) <= 1.0e-8
