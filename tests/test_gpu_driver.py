@@ -148,7 +148,7 @@ def small(qa, orc):
 @pytest.mark.parametrize("T", [5, 156, 1024])
 def test_nocache_entry_points_match_oracle(qa, small, T):
     """qa_decoder_layer_forward_nocache and qa_decoder_prefill_nocache (positions 0..T-1, f32 K/V never
-    stored) at T = 5 (skinny MFMA projections), 156 and 1024 (rocBLAS projections), against
+    stored) at T = 5 (skinny MFMA projections), 156 and 1024 (prompt GEMM), against
     orc_layer_forward_nocache / the oracle's non-cached prefill; the cache is left untouched."""
     model, om = small
     x = qa.prompt_input(model, T - 3, 3)

@@ -450,11 +450,12 @@ def test_prefill_attention_exact_two_pass(qa):
 PF_FIXED = 4096 + 8192 * 256
 
 
-@pytest.mark.parametrize("n_past,T", [(0, 1500), (600, 1500)])
+@pytest.mark.parametrize("n_past,T", [(0, 1500), (600, 1500), (0, 2500), (600, 2430), (3000, 1100)])
 def test_prefill_split_and_unsplit_agree(qa, orc, n_past, T):
     """The longest query tiles cut in two parts (full workspace) and one item per tile (a workspace
     with room for the statistics only) both match the oracle; repeated calls sharing one workspace,
-    with other shapes in between, give identical bits (queue and merge counters return to zero)."""
+    with other shapes in between, give identical bits (queue and merge counters return to zero).  Up to 2176
+    positions the key groups serve the call, which use neither; the larger ones run on the 128-token tiles."""
     L = n_past + T
     lay = layout(qa, 1, 1, L + 3, True)
     cache = Cache(qa, lay)
@@ -474,10 +475,11 @@ def test_prefill_split_and_unsplit_agree(qa, orc, n_past, T):
         print(f"prefill {label} n_past={n_past} T={T}", flush=True)
         qa.check(qa.lib.qa_prefill_attn(d_q.ptr, cache.ptr, C.byref(lay), 0, 0, n_past, T, 16, SCALE, d_out.ptr,
                                         ws.ptr, nbytes, NULL_STREAM))
-        # another shape on the same workspace in between
-        d_o2 = zeros(qa, (37, 2048))
-        qa.check(qa.lib.qa_prefill_attn(d_q.ptr, cache.ptr, C.byref(lay), 0, 0, 5, 37, 16, SCALE, d_o2.ptr,
-                                        ws.ptr, full, NULL_STREAM))
+        # other shapes on the same workspace in between, on both kernels
+        d_o2 = zeros(qa, (T, 2048))
+        for past2, T2 in [(5, 37)] + ([(5, min(T, 2190)), (L - 130, 129)] if L > 2200 else []):
+            qa.check(qa.lib.qa_prefill_attn(d_q.ptr, cache.ptr, C.byref(lay), 0, 0, past2, T2, 16, SCALE, d_o2.ptr,
+                                            ws.ptr, full, NULL_STREAM))
         qa.synchronize()
         outs[label] = d_out.numpy().reshape(T, 16, 128)
         check_close(outs[label], ref)

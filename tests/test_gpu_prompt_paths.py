@@ -1,0 +1,119 @@
+"""Paths around the prompt GEMM that the other tests do not reach: f32 weights without its copies (skinny MFMA GEMM up to
+64 rows, rocBLAS beyond), shapes it does not take and shapes of odd 64-k counts, steps of more than 32 streams, and NaN in
+the f16 key groups."""
+import ctypes as C
+import os
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _gpu(qa):
+    assert qa.device_count() > 0, "no HIP device: GPU tests need the MI355X"
+
+
+def _without_copies(make):
+    os.environ["QA_PROMPT_COPIES"] = "0"
+    try:
+        return make()
+    finally:
+        del os.environ["QA_PROMPT_COPIES"]
+
+
+def _layers_match(dec, om, x, T, cached, capacity):
+    """Four projections in a row, f32 sums in another order: 1.4e-5 of a layer (relative 2-norm)."""
+    if cached:
+        got, ref = dec.layer_forward(0, x[:T], 0), om.layer_forward_cached(0, x[:T], 0, om.cache(capacity, False))
+    else:
+        got, ref = dec.layer_forward_nocache(0, x[:T]), om.layer_forward_nocache(0, x[:T])
+    d = got.astype(np.float64) - ref
+    assert np.linalg.norm(d) <= 1.4e-5 * np.linalg.norm(ref), (T, np.linalg.norm(d) / np.linalg.norm(ref))
+
+
+LENGTHS = (5, 40, 64, 65, 156, 300)
+
+
+@pytest.mark.parametrize("cached", [False, True], ids=["nocache", "cached"])
+def test_f32_weights_without_copies(qa, orc, cached):
+    model = qa.Model(qa.QWEN3_ASR_0_6B, n_layers=1)
+    om = orc.OracleModel.from_product_model(model)
+    x = qa.prompt_input(model, 290, 10)
+    with _without_copies(lambda: qa.Decoder(model, 1, 300, qa.QA_CACHE_F32)) as dec:
+        for T in LENGTHS:
+            print(f"no copies, T={T}", flush=True)
+            _layers_match(dec, om, x, T, cached, 300)
+
+
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32-weights", "bf16-copies"])
+@pytest.mark.parametrize("hidden,intermediate", [(960, 992), (640, 1984), (128, 64)])
+def test_other_shapes(qa, orc, hidden, intermediate, bf16):
+    """960 / 992 are no multiples of 128 and 64: the whole prompt runs on the f32 GEMMs.  640 / 1984: K of 10 and 31
+    blocks of 64, which no K group or slice divides evenly and whose last block of 256 is cut; 128 / 64: one or two."""
+    size = qa.ModelSize("other", hidden=hidden, intermediate=intermediate, n_layers=1, vocab=1024)
+    model = qa.Model(size, n_layers=1, bf16=bf16)
+    om = orc.OracleModel.from_product_model(model)
+    x = qa.prompt_input(model, 690, 10)
+    with qa.Decoder(model, 1, 700, qa.QA_CACHE_F32) as dec:
+        assert dec.weights_bf16 == bf16
+        for T in LENGTHS + (700,):
+            print(f"hidden {hidden} intermediate {intermediate} bf16={bf16} T={T}", flush=True)
+            _layers_match(dec, om, x, T, True, 700)
+
+
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32-weights", "bf16-copies"])
+@pytest.mark.parametrize("n_streams", [33, 40])
+def test_more_than_32_streams(qa, orc, greedy, n_streams, bf16):
+    """Steps of more than 32 streams run the prompt projections, each stream at its own position, against the oracle
+    decoding each stream alone."""
+    from qwenasr_amd import configs
+
+    model = qa.Model(qa.QWEN3_ASR_0_6B, n_layers=1, vocab=8192, bf16=bf16)
+    om = orc.OracleModel.from_product_model(model)
+    rng = np.random.default_rng(n_streams)
+    lens = rng.integers(20, 180, n_streams)
+    first = rng.integers(0, model.cfg.vocab, n_streams).astype(np.int32)
+    steps, cap = 3, 200
+    with qa.Decoder(model, n_streams, cap, qa.QA_CACHE_F16) as dec:
+        refs = []
+        for s in range(n_streams):
+            k, v = configs.cfg4_stream_kv(1000 + s, int(lens[s]), n_layers=1)
+            dec.fill_cache(s, k, v, int(lens[s]))
+            cache = om.cache(cap, True)
+            cache.fill(k, v, int(lens[s]))
+            refs.append([list(r) for r in om.decode_steps(cache, int(first[s]), steps)])
+        print(f"{n_streams} streams: oracle done", flush=True)
+        got = dec.decode_streams(first, steps)
+        for s in range(n_streams):
+            greedy.match(got[:, s].tolist(), *refs[s], f"{n_streams}-stream step, {'bf16' if bf16 else 'f32'} weights, stream {s}")
+        assert dec.device_lens().tolist() == (lens + steps).tolist()
+
+
+@pytest.mark.parametrize("T,bad", [(33, 32), (129, 96), (300, 32), (2300, 64)])
+def test_f16_prefill_keeps_nan(qa, T, bad):
+    """As the f32 kernel's test: a NaN in key row `bad` of KV head 3 reaches every query of that head that attends it,
+    the key groups (T up to 2176) and the 128-token tiles alike; nothing else moves by a bit."""
+    rng = np.random.default_rng(T + bad)
+    q = qa.DeviceArray.from_numpy(rng.standard_normal((T, 2048)).astype(np.float32))
+    kv = rng.standard_normal((2, 8, T, 128)).astype(np.float16)
+    lay = qa.KvLayout(1, 1, 8, 128, T, qa.QA_CACHE_F16)
+    nbytes = qa.lib.qa_prefill_attn_workspace_bytes(T, 16)
+    ws = qa.DeviceArray((nbytes,), np.uint8)
+    outs = []
+    for poisoned in (False, True):
+        if poisoned:
+            kv[0, 3, bad, 17] = np.nan
+        cache, out = qa.DeviceArray.from_numpy(kv), qa.DeviceArray((T, 2048))
+        print(f"f16 prefill T={T} NaN key {bad if poisoned else None}", flush=True)
+        qa.check(qa.lib.qa_prefill_attn(q.ptr, cache.ptr, C.byref(lay), 0, 0, 0, T, 16, 128 ** -0.5, out.ptr, ws.ptr, nbytes,
+                                        None))
+        qa.synchronize()
+        outs.append(out.numpy().reshape(T, 16, 128))
+    clean, got = outs
+    assert np.isfinite(clean).all()
+    hit = np.zeros(clean.shape, bool)
+    hit[bad:, 6:8] = True
+    assert np.isnan(got[hit]).all()
+    np.testing.assert_array_equal(got[~hit].view(np.uint32), clean[~hit].view(np.uint32))
