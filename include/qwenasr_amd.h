@@ -180,7 +180,8 @@ int qa_decode_noalloc_prepare(void);
 /* Causal prefill attention over the cache (row a7): the n_tokens queries of stream `stream_idx` at
  * positions n_past .. n_past + n_tokens - 1, query t attending keys [0, n_past + t].  Same
  * arithmetic as qa_decode_attn.  f16 caches run on CDNA4 f16 MFMA: one pass over work items pulled
- * from per-KV-head queues (QA_PREFILL_EXACT=1: row statistics, then p and PV), short prompts one launch without them.
+ * from per-KV-head queues (QA_PREFILL_EXACT=1: row statistics, then p and PV); short prompts, and
+ * chunks of up to 1024 tokens behind cached positions, run without the queues.
  * workspace (f16 caches): qa_prefill_attn_workspace_bytes(n_tokens, n_heads) bytes, cleared once
  * with qa_workspace_clear before the first call; it holds the queue and merge counters (every call
  * leaves them zero, so one workspace serves any sequence of calls with at most n_tokens tokens),
@@ -237,8 +238,9 @@ int qa_gemm_rows_fused_bf16(const uint16_t * W_bf16, int32_t out_dim, int32_t in
                             float * y, int32_t accumulate, const float * norm_w, const double * stats_in,
                             int32_t n_stats_in, float eps, double * stats_out, int32_t swiglu,
                             void * workspace, size_t workspace_bytes, void * stream);
-/* GEMM on bf16-exact weights for many rows, replacing linear_ggml (text-decoder.cpp:83-90) on a split input  *
- * (the decoder's own prompts run another kernel, gemm_prefill.hip): x_split = [rows][3 in_dim] bf16 bits, each row the three-part split [hi | mid | lo] of an f32  *
+/* GEMM on bf16-exact weights for many rows, replacing linear_ggml (text-decoder.cpp:83-90) on a split  *
+ * input that the caller makes (the decoder's own prompts run another kernel, gemm_prefill.hip):         *
+ * x_split = [rows][3 in_dim] bf16 bits, each row the three-part split [hi | mid | lo] of an f32         *
  * input row (x = hi + mid + lo exactly), and y[rows][out_dim] (+)= sum of the three parts times W^T:    *
  * exact f32 products, f32 sums (bf16 MFMA).  in_dim % 64 == 0, out_dim % 256 == 0.  With act_split    *
  * != NULL (y NULL, accumulate 0) W_bf16 = [gate rows; up rows] (2 out_dim rows, out_dim % 128 == 0)    *

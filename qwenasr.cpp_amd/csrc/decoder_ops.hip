@@ -778,7 +778,8 @@ struct GemmRowsPlan {
 };
 
 // tuning overrides of the <= 32-row plan: QA_GR32_WGS (workgroup target, default 256) and QA_GR32_DEPTH
-// (blocks in flight per wave, 1 or 2)
+// (blocks in flight per wave, 1 or 2: f32 weights, and bf16 weights with two 32-row tiles per workgroup; the other bf16
+// kernels have one)
 int env_int(const char * name, int fallback) {
     const char * e = std::getenv(name);
     return e ? std::atoi(e) : fallback;

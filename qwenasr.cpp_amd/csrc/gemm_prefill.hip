@@ -11,10 +11,10 @@
 // zeros, and both forms follow one plan and one order, so f32 weights that hold bf16 values give the bits of their bf16
 // copies.
 //
-// Sums.  The bf16 MFMA rounds its sums down a little more often than up (a mean of 2 to 10% of a last place, whatever the
-// sign), and six MFMAs per 16 k on f32 weights add up to -1.1e-7 of the outputs' root mean square over 2048 k: the same
+// Sums.  The bf16 MFMA rounds a sum down more often than up, whatever its sign (products as large as the sum: 41% down,
+// 31% up), and six MFMAs per 16 k on f32 weights add up to -1.1e-7 of the outputs' root mean square over 2048 k: the same
 // for every token, so an average over tokens, as the attention takes, keeps it while it loses the signal.  X is therefore
-// stored negated in every second pair of blocks of 256 k (split_negated), and the accumulators turn round with it: 1e-9.
+// stored negated in blocks + - - + of 256 k (split_negated), and the accumulators turn round with it: 1e-9 remains.
 // Up to 64 tokens (SUMS) every block of 256 k is a sum of its own, as short as the chains of the f32 kernel before.
 // Relative error against float64 (2-norm, N(0, 1) rows): q|k|v of 2048 k 1.9e-7 at 33 to 64 tokens (gemm_rows_kernel
 // 2.0-2.2e-7), 3.5e-7 at 156 and 6.9e-7 from 700 on (sgemm 8.1e-7); a 1.7B layer whose residual is scaled away 0.72-0.77e-6
@@ -29,12 +29,13 @@
 // Work split.  A workgroup is wm token tiles x kw K groups of waves over 128 columns and one of ks K slices
 // (prompt_plan); K groups are summed through LDS, K slices are left as partial sums that the next row kernel adds
 // up in slice order (prompt_norm, prompt_swiglu, the append), so no workgroup waits for another.
-// What bounds it: at T = 156 a 1.7B layer's four GEMMs take 75 us on bf16 weights, against 39 us of MFMA time at 1.2
-// PFLOP/s and 16 us for the 100 MB of weights; short K slices are chains of first loads, 4-16 stages and a tail.
-// (The 128 x 256 tiles of gemm_split3.hip put 16-96 workgroups on 256 CUs: 415 us; gemm_rows_kernel on f32 weights
-// 296 us at T = 52, now 45.)  On f32 weights 126 us (229 with rocBLAS sgemm).  At T = 3913 it runs at 1.06-1.27
-// PFLOP/s, the rate power allows (a library bf16 GEMM of random operands: 1.2): 1046 us per layer on bf16 weights
-// (gemm_split3.hip 1045), 1921 us on f32 weights (sgemm 3092, at 98% of the f32 MFMA rate).
+// What bounds it (us of a 1.7B layer's four GEMMs, traced in whole calls, weights from HBM): at T = 156 96 on bf16 weights,
+// against 39 of MFMA time at 1.2 PFLOP/s and 16 for the 100 MB of weights; short K slices are chains of first loads, 4-16
+// stages and a tail.  (The 128 x 256 tiles of gemm_split3.hip put 16-96 workgroups on 256 CUs: 436; at T = 52
+// gemm_rows_kernel on f32 weights 294, now 59.)  f32 weights: T = 52 91 (gemm_rows_kernel 293), T = 156 166 (rocBLAS sgemm
+// 259).  At T = 3913 it executes 1.16-1.21 PFLOP/s, the rate power allows (a library bf16 GEMM of random operands: 1.2),
+// with the matrix cores busy for 0.5 to 0.64 of the cycles: 1065 on bf16 weights (gemm_split3.hip 1103), 2044 on f32 weights
+// (sgemm 2892, at 98% of the f32 MFMA rate).
 #include "ops.hpp"
 #include "split3.hpp"
 #include "wave.hpp"
@@ -626,8 +627,10 @@ int prompt_norm_launch(float * x, const float * partial, int32_t slices, const f
     if (!x || rows <= 0 || dim <= 0 || dim % 16 || dim > 8192 || (Xf && !w) || (slices > 0 && !partial)) {
         return fail(QA_ERR_INVALID, "prompt_norm: invalid arguments");
     }
-    // R = 8 from two workgroups per CU on (3913 rows of 2048: 21 against 40 us; 156 rows: 9 against 6)
-    const bool r8 = rows >= 4096 / 4 && dim <= 2048;
+    // R = 8 from 1024 rows (128 workgroups) on; below, one row per workgroup keeps more loads in flight.  us R 1 / R 8:
+    // rows of 2048 156 6 / 9, 1000 14.0 / 14.1, 1200 15.6 / 13.3, 3913 40 / 21; rows of 1024 1000 9.6 / 10.9, 1200 9.6 / 9.4,
+    // 1500 11.1 / 8.8
+    const bool r8 = rows >= 1024 && dim <= 2048;
     const dim3 grid(static_cast<unsigned>(r8 ? (rows + 7) / 8 : rows)), block(r8 ? 512 : 256);
 #define QA_NORM(R, IT) hipLaunchKernelGGL((prompt_norm_kernel<R, IT>), grid, block, 0, stream, x, partial, slices, w, rows, dim, eps, Xf)
     if (r8 && dim <= 1024) QA_NORM(8, 2);
