@@ -388,7 +388,10 @@ int qa_wav_info(const char * path, int64_t * n_samples, int32_t * sample_rate);
 /* ---------------------------------------------------------------- runtime layer */
 typedef struct qa_decoder qa_decoder;
 
-/* Uploads the weights, allocates the cache (zeroed) and workspaces on device 0. */
+/* Uploads the weights, allocates the cache (zeroed) and workspaces on device 0.  With f32 weights it    *
+ * then lays out split copies of the layer weights for prompts (6 bytes per weight) while as much memory *
+ * again stays free; a later allocation of the decoder that fails takes them back.  QA_PROMPT_COPIES=0   *
+ * at creation declines them.                                                                            */
 int qa_decoder_create(const qa_text_config * cfg, const qa_model_weights * weights, int32_t n_streams,
                       int32_t max_seq, int32_t cache_type, qa_decoder ** out);
 void qa_decoder_destroy(qa_decoder * dec);
