@@ -222,6 +222,14 @@ int32_t prompt_min_rows(const qa_decoder * d) {
     return !prompt_ready(d) ? INT32_MAX : d->layers[0].qkv16 ? 2 : 33;
 }
 
+// A step of 65 to 128 streams on f32 weights of at most 1024 hidden units keeps sgemm: its one tile of 128 rows is as fast
+// there, and around the decode attention, which takes whole rows and gives whole rows, the prompt GEMM needs two launches
+// more per layer (4 layers, us, sgemm / prompt GEMM: 65 streams 394 / 440, 128 429 / 486, 64 629 (gemm_rows_kernel) / 417,
+// 160 631 / 550; hidden 2048: 1116 / 647, 1136 / 714).
+bool step_on_sgemm(const qa_decoder * d, int32_t rows) {
+    return !d->layers[0].qkv16 && d->cfg.hidden <= 1024 && rows > kSkinnyRows && rows <= 128;
+}
+
 // Gives the prompt copies of f32 weights back after an allocation failed; the activations are laid out again by the
 // next ensure_rows (prompts then run on sgemm, which needs other buffers).
 bool drop_prompt_copies(qa_decoder * d) {
@@ -247,7 +255,8 @@ int alloc_rows(qa_decoder * d, int32_t rows) {
     rc = rc ? rc : dmalloc_t(d->act_allocs, R * (QD + 2 * KD), &d->qkv);
     rc = rc ? rc : dmalloc_t(d->act_allocs, R * QD, &d->qrot);
     rc = rc ? rc : dmalloc_t(d->act_allocs, R * QD, &d->attn);
-    const size_t gu_rows = std::min(rows, prompt_min_rows(d) - 1);   // rows that do not run the prompt GEMMs
+    // rows that do not run the prompt GEMMs
+    const size_t gu_rows = std::max(std::min(rows, prompt_min_rows(d) - 1), step_on_sgemm(d, d->n_streams) ? d->n_streams : 0);
     if (gu_rows >= 2) rc = rc ? rc : dmalloc_t(d->act_allocs, gu_rows * 2 * I, &d->gu);
     rc = rc ? rc : dmalloc_t(d->act_allocs, R * I, &d->act);
     // the LM head runs on one row per stream (decode) or the last row (prefill)
@@ -386,7 +395,7 @@ int run_layer(qa_decoder * d, int32_t l, int32_t rows, int kind, int32_t n_past,
     const int32_t H = c.hidden, QD = c.n_heads * kHeadDim, KD = c.n_kv_heads * kHeadDim, I = c.intermediate;
     const int32_t W3 = QD + 2 * KD;
     hipStream_t s = d->stream;
-    const bool prompt = !fused && d->xf && rows >= prompt_min_rows(d);
+    const bool prompt = !fused && d->xf && rows >= prompt_min_rows(d) && !(kind == kDecode && step_on_sgemm(d, rows));
     int32_t slices = 0;        // K slices of the q|k|v projection, still partial sums in d->partial
     bool attn_split = false;   // the attention left its output split in d->xf
     int rc;

@@ -3,6 +3,7 @@
 the f16 key groups."""
 import ctypes as C
 import os
+import time
 
 import numpy as np
 import pytest
@@ -64,10 +65,12 @@ def test_other_shapes(qa, orc, hidden, intermediate, bf16):
 
 
 @pytest.mark.parametrize("bf16", [False, True], ids=["f32-weights", "bf16-copies"])
-@pytest.mark.parametrize("n_streams", [33, 40])
-def test_more_than_32_streams(qa, orc, greedy, n_streams, bf16):
-    """Steps of more than 32 streams run the prompt projections, each stream at its own position, against the oracle
-    decoding each stream alone."""
+@pytest.mark.parametrize("n_streams", [33, 40, 65, 129])
+def test_more_than_32_streams(qa, orc, n_streams, bf16):
+    """Steps of more than 32 streams run the prompt projections (65 to 128 on f32 weights of this size: sgemm), each stream
+    at its own position, against the oracle decoding each stream alone.  Logits of rms 0.64 (embeddings N(0, 0.02), hidden
+    1024) over f16 caches are off by up to 2.5e-4 of it in the 2-norm, four times that in one of 8192: ids may part only
+    where the oracle's two best are closer than twice 6.4e-4, and then the runner-up is taken."""
     from qwenasr_amd import configs
 
     model = qa.Model(qa.QWEN3_ASR_0_6B, n_layers=1, vocab=8192, bf16=bf16)
@@ -86,9 +89,38 @@ def test_more_than_32_streams(qa, orc, greedy, n_streams, bf16):
             refs.append([list(r) for r in om.decode_steps(cache, int(first[s]), steps)])
         print(f"{n_streams} streams: oracle done", flush=True)
         got = dec.decode_streams(first, steps)
+        ties = 0
         for s in range(n_streams):
-            greedy.match(got[:, s].tolist(), *refs[s], f"{n_streams}-stream step, {'bf16' if bf16 else 'f32'} weights, stream {s}")
+            ids, margins, runner = refs[s]
+            parts = [i for i in range(steps) if got[i, s] != ids[i]][:1]    # after it the streams are fed different ids
+            assert all(margins[i] < 1.3e-3 and got[i, s] == runner[i] for i in parts), (s, parts, got[:, s], ids, margins)
+            ties += len(parts)
+        print(f"{n_streams} streams: {ties} near-ties", flush=True)
+        assert ties <= 2
         assert dec.device_lens().tolist() == (lens + steps).tolist()
+
+
+def test_steps_of_65_to_128_streams_keep_sgemm(qa):
+    """On f32 weights of hidden 1024 a step of 65 streams is 12% slower on the prompt GEMM than on sgemm: with the weights'
+    copies it takes what it takes without them."""
+    model = qa.Model(qa.QWEN3_ASR_0_6B, n_layers=4, vocab=8192)
+    streams = 65
+    decoders = [qa.Decoder(model, streams, 160, qa.QA_CACHE_F16),
+                _without_copies(lambda: qa.Decoder(model, streams, 160, qa.QA_CACHE_F16))]
+    first = np.arange(streams, dtype=np.int32)
+    us = [[], []]
+    for _ in range(9):
+        for i, dec in enumerate(decoders):
+            for s in range(streams):
+                qa.check(qa.lib.qa_decoder_set_cur_len(dec.handle, s, 100))
+            t = time.perf_counter()
+            dec.decode_streams(first, 30)
+            us[i].append((time.perf_counter() - t) / 30 * 1e6)
+    a, b = (sorted(v)[3] for v in us)
+    print(f"65 streams: {a:.1f} us a step, {b:.1f} us without the copies", flush=True)
+    for dec in decoders:
+        dec.close()
+    assert a < 1.05 * b
 
 
 @pytest.mark.parametrize("T,bad", [(33, 32), (129, 96), (300, 32), (2300, 64)])
