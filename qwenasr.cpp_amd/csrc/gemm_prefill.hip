@@ -15,7 +15,8 @@
 // 31% up), and six MFMAs per 16 k on f32 weights add up to -1.1e-7 of the outputs' root mean square over 2048 k: the same
 // for every token, so an average over tokens, as the attention takes, keeps it while it loses the signal.  X is therefore
 // stored negated in blocks + - - + of 256 k (split_negated), and the accumulators turn round with it: 1e-9 remains.
-// Up to 64 tokens (SUMS) every block of 256 k is a sum of its own, as short as the chains of the f32 kernel before.
+// At 33 to 64 tokens (SUMS) every block of 256 k is a sum of its own, as short as the chains of the f32 kernel before,
+// where a wave sums over more than one.
 // Relative error against float64 (2-norm, N(0, 1) rows): q|k|v of 2048 k 1.9e-7 at 33 to 64 tokens (gemm_rows_kernel
 // 2.0-2.2e-7), 3.5e-7 at 156 and 6.9e-7 from 700 on (sgemm 8.1e-7); a 1.7B layer whose residual is scaled away 0.72-0.77e-6
 // (0.77-0.79e-6), 1.5e-6 at 156 and 2.3-2.6e-6 from 700 on (sgemm 2.8-3.0e-6; without the negation 2.9-4.2e-6).
@@ -548,10 +549,16 @@ int launch_wm(const PgParams & p, int nt, hipStream_t stream) {
     }
     switch (p.wm) {
         case 2:
-            // the sums of short blocks for up to 64 tokens, where f32 weights had sums as short before; with more groups of
-            // tokens one workgroup per CU, as their registers ask for, costs more than it brings (f32 weights, whole calls
-            // of 4 layers: 100 tokens 899 / 912 us, 300 tokens 1451 / 1483)
-            return p.m_groups == 1 ? launch_one<WP, EPI, 4, B / 2, true>(p, stream) : launch_one<WP, EPI, 4, B / 2>(p, stream);
+            // Sums of blocks of 256 k where f32 weights had sums as short before, 33 to 64 tokens, and a wave's k reach over
+            // more than one block (1.7B: gate|up 512 k, down 192; a length that divides 256 stays in one).  With more groups
+            // of tokens one workgroup per CU, as their registers ask for, costs more than it brings (f32 weights, whole calls
+            // of 4 layers: 100 tokens 899 / 912 us, 300 tokens 1451 / 1483).  Up to 32 tokens only bf16 weights come
+            // here: without, 14 tokens are off by 0.60e-6 (with 0.55, f32 kernels 0.77; a 1.7B layer whose residual is scaled
+            // away) and calls of 4 layers take 2% less (20 tokens, 0.6B: 366 us, with 373).
+            if (p.m_tiles == 2 && p.m_groups == 1 && kSplitSign % (p.per * 16 * Stage<WP, 4>::kSteps) != 0) {
+                return launch_one<WP, EPI, 4, B / 2, true>(p, stream);
+            }
+            return launch_one<WP, EPI, 4, B / 2>(p, stream);
         case 3: return launch_one<WP, EPI, 4, (B + 2) / 3>(p, stream);
         case 4: return launch_one<WP, EPI, 4, B / 4>(p, stream);
         case 5: return launch_one<WP, EPI, 4, (B + 4) / 5>(p, stream);
